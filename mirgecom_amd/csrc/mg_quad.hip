@@ -5,6 +5,7 @@
 #include <mutex>
 #include <string>
 
+#include "mg_esdg_pairs.h"
 #include "mgdg_host.h"
 
 extern "C" {
@@ -115,13 +116,99 @@ mg_status esdg_check(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* quad
   return MG_OK;
 }
 
+constexpr size_t kEsdgBudget = 128 * 1024;
+
+// The paired flux-differencing kernels (mg_esdg_pairs.h) take 3-D elements
+// with the default quadrature (their lane layout is its point counts) and the
+// operators' cyclic diagonals; any other rule goes row by row, which evaluates
+// nearly every two-point flux twice.
+template <int D, int P>
+bool esdg_paired(const mgdg::EsdgArgs& ea) {
+  if constexpr (D == 3) {
+    using C = mgdg::EsdgPairs<P, false>;
+    return ea.skew_diag && ea.ext_diag && ea.nq == C::NQ && ea.nfq == C::NFQ;
+  } else {
+    return false;
+  }
+}
+
+template <typename Kern>
+mg_status esdg_launch_one(Kern kern, const char* name, size_t lds, size_t budget, int epb,
+                          const mgdg::KArgs& a, mgdg::EsdgArgs& ea, hipStream_t st) {
+  mg_status s = set_lds(kern, budget);
+  if (s) return s;
+  ea.epb = epb;
+  hipLaunchKernelGGL(kern, dim3(unsigned((a.K + epb - 1) / epb)), dim3(mgdg::kBlock), lds, st,
+                     a, ea);
+  return check_launch(name);
+}
+
+template <typename Kern>
+mg_status esdg_launch_project(Kern kern, const char* name, int nfld, const mgdg::KArgs& a,
+                              mgdg::EsdgArgs& ea, hipStream_t st) {
+  const size_t per = sizeof(double) * nfld * ea.nq;
+  if (per > kEsdgBudget) return fail(MG_ERR_UNSUPPORTED, "quadrature too large for LDS");
+  const int epb = std::max(1, std::min(8, 256 / ea.nq));
+  return esdg_launch_one(kern, name, per * epb, kEsdgBudget, epb, a, ea, st);
+}
+
+// Row-by-row kernels: as many elements as fit 64 KiB, at most 16.
+template <typename Kern>
+mg_status esdg_launch_rows(Kern kern, const char* name, size_t per, const mgdg::KArgs& a,
+                           mgdg::EsdgArgs& ea, hipStream_t st) {
+  if (per > kEsdgBudget) return fail(MG_ERR_UNSUPPORTED, "quadrature too large for LDS");
+  const int epb = int(std::max<size_t>(1, std::min<size_t>(16, (64 * 1024) / per)));
+  return esdg_launch_one(kern, name, per * epb, kEsdgBudget, epb, a, ea, st);
+}
+
+template <int D, int P, int NS>
+mg_status esdg_launch(const mgdg::KArgs& a, mgdg::EsdgArgs& ea, hipStream_t st) {
+  using E = mgdg::Elem<D, P>;
+  mg_status s = esdg_launch_project(mgdg::esdg_project_kernel<D, P, NS>,
+                                    "esdg_project_kernel", 2 + D + NS, a, ea, st);
+  if (s) return s;
+  if constexpr (D == 3) {
+    if (esdg_paired<D, P>(ea)) {
+      constexpr size_t lds = mgdg::EsdgPairCfg<P, NS>::LDS;
+      return esdg_launch_one(mgdg::esdg_pair_kernel<P, NS>, "esdg_pair_kernel", lds, lds,
+                             mgdg::EsdgPairs<P, false>::EPB, a, ea, st);
+    }
+  }
+  const size_t nq = ea.nq, nft = size_t(D + 1) * ea.nfq, nh = ea.nh;
+  const size_t nacc = (nh + nq - 1) / nq * nq + nft;
+  const size_t per = sizeof(mgdg::EcPairLog<D, NS>) * nh +
+                     sizeof(double) * (2 + D + NS) * (2 * E::NP + E::NFN + nft + nacc);
+  return esdg_launch_rows(mgdg::esdg_kernel<D, P, NS>, "esdg_kernel", per, a, ea, st);
+}
+
+template <int D, int P>
+mg_status esdg_mix_launch(const mgdg::KArgs& a, mgdg::EsdgArgs& ea, hipStream_t st) {
+  using E = mgdg::Elem<D, P>;
+  constexpr int NF = 2 + D + mgdg::MIX_NSP;
+  mg_status s = esdg_launch_project(mgdg::esdg_project_mix_kernel<D, P>,
+                                    "esdg_project_mix_kernel", NF, a, ea, st);
+  if (s) return s;
+  if constexpr (D == 3) {
+    if (esdg_paired<D, P>(ea)) {
+      constexpr size_t lds = mgdg::EsdgMixCfg<P>::LDS;
+      return esdg_launch_one(mgdg::esdg_mix_pair_kernel<P>, "esdg_mix_pair_kernel", lds, lds,
+                             mgdg::EsdgPairs<P, true>::EPB, a, ea, st);
+    }
+  }
+  const size_t nq = ea.nq, nft = size_t(D + 1) * ea.nfq, nh = ea.nh;
+  const size_t nacc = (nh + nq - 1) / nq * nq + nft;
+  const size_t per = sizeof(mgdg::RnPair<D>) * nh +
+                     sizeof(double) * (NF * (2 * E::NP + E::NFN + nft + nacc) + 2 * E::NP +
+                                       E::NFN + 2 * nft);
+  return esdg_launch_rows(mgdg::esdg_mix_kernel<D, P>, "esdg_mix_kernel", per, a, ea, st);
+}
+
 mg_status esdg_run(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* quad,
                    const mg_esdg* esdg, const double* q, const double* q_bnd_quad,
                    int32_t dissipation, double* ev_work, double* rhs, void* stream) {
   mg_status s = esdg_check(mesh, gas, quad, esdg, q, q_bnd_quad, rhs);
   if (s) return s;
   if (!ev_work) return fail(MG_ERR_ARG, "ev_work NULL");
-  const int nfld = 2 + mesh->dim + gas->nspecies;
   mgdg::KArgs a = make_args(mesh, gas);
   a.q = q;
   a.out = rhs;
@@ -144,40 +231,10 @@ mg_status esdg_run(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* quad,
   ea.dissipation = dissipation ? 1 : 0;
   ea.skew_diag = esdg->skew_diag;
   ea.ext_diag = esdg->ext_diag;
-  ea.paired = (mesh->dim == 3 && quad->nq == 64 && mesh->nfaces * quad->nfq == 192 &&
-               esdg->skew_diag && esdg->ext_diag && mgdg::kBlock == 256)
-                  ? 1
-                  : 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  constexpr size_t kBudget = 128 * 1024;
-  const size_t nft = size_t(mesh->nfaces) * quad->nfq;
-#define MG_ECASE(D, P, NS)                                                              \
-  if (mesh->dim == D && mesh->order == P && gas->nspecies == NS) {                      \
-    const size_t per_p = sizeof(double) * nfld * quad->nq;                              \
-    if (per_p > kBudget) return fail(MG_ERR_UNSUPPORTED, "quadrature too large for LDS"); \
-    int epb_p = int(std::max<size_t>(1, std::min<size_t>(8, 256 / quad->nq)));        \
-    ea.epb = epb_p;                                                                     \
-    auto kp = mgdg::esdg_project_kernel<D, P, NS>;                                      \
-    if ((s = set_lds(kp, kBudget))) return s;                                           \
-    hipLaunchKernelGGL(kp, dim3(unsigned((a.K + epb_p - 1) / epb_p)),                   \
-                       dim3(mgdg::kBlock), per_p * epb_p, st, a, ea);                  \
-    if ((s = check_launch("esdg_project_kernel"))) return s;                            \
-    const size_t nchunk = (size_t(esdg->nh) + quad->nq - 1) / quad->nq;               \
-    const size_t nacc = std::max(nchunk * quad->nq + nft, nft);                         \
-    const size_t per_e = sizeof(mgdg::EcPair<D, NS>) * esdg->nh +                       \
-        sizeof(double) * nfld *                                                         \
-            (2 * size_t(mesh->np) + size_t(mesh->nfaces) * mesh->nfp +                  \
-             (ea.paired ? 0 : nft) + nacc);                                             \
-    if (per_e > kBudget) return fail(MG_ERR_UNSUPPORTED, "quadrature too large for LDS"); \
-    int epb = ea.paired ? 1                                                             \
-                        : int(std::max<size_t>(1, std::min<size_t>(16, (64 * 1024) / per_e))); \
-    ea.epb = epb;                                                                       \
-    auto kern = mgdg::esdg_kernel<D, P, NS>;                                            \
-    if ((s = set_lds(kern, kBudget))) return s;                                         \
-    hipLaunchKernelGGL(kern, dim3(unsigned((a.K + epb - 1) / epb)), dim3(mgdg::kBlock), \
-                       per_e * epb, st, a, ea);                                         \
-    return check_launch("esdg_kernel");                                                 \
-  }
+#define MG_ECASE(D, P, NS)                                              \
+  if (mesh->dim == D && mesh->order == P && gas->nspecies == NS)          \
+    return esdg_launch<D, P, NS>(a, ea, st);
   MG_ECASE(2, 1, 0) MG_ECASE(2, 2, 0) MG_ECASE(2, 3, 0) MG_ECASE(2, 4, 0)
   MG_ECASE(3, 1, 0) MG_ECASE(3, 2, 0) MG_ECASE(3, 3, 0)
   MG_ECASE(2, 1, 7) MG_ECASE(2, 2, 7) MG_ECASE(2, 3, 7) MG_ECASE(2, 4, 7)
@@ -191,7 +248,7 @@ mg_status esdg_run(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* quad,
 }
 
 // The uiuc_7sp mixture (Renac's two-point flux): esdg_project_mix_kernel
-// then esdg_mix_kernel (row-by-row phase 4).
+// then esdg_mix_kernel.
 mg_status esdg_mix_run(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* quad,
                        const mg_esdg* esdg, const double* q, const double* temperature,
                        const double* q_bnd_quad, const double* t_bnd_quad, int32_t niter,
@@ -215,7 +272,6 @@ mg_status esdg_mix_run(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* qu
   if (mesh->nbnd_nodes > 0 && (!q_bnd_quad || !t_bnd_quad))
     return fail(MG_ERR_ARG, "boundary exterior state / temperature missing");
   if (mesh->nbnd_nodes % mesh->nfp) return fail(MG_ERR_ARG, "nbnd_nodes % nfp");
-  const int nfld = 2 + mesh->dim + gas->nspecies;
   mgdg::KArgs a = make_args(mesh, gas);
   a.q = q;
   a.temp = temperature;
@@ -240,36 +296,11 @@ mg_status esdg_mix_run(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* qu
   ea.dissipation = dissipation ? 1 : 0;
   ea.niter = niter;
   ea.es_volume = es_volume ? 1 : 0;
-  ea.paired = 0;
+  ea.skew_diag = esdg->skew_diag;
+  ea.ext_diag = esdg->ext_diag;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  constexpr size_t kBudget = 128 * 1024;
-  const size_t nft = size_t(mesh->nfaces) * quad->nfq;
-  const size_t nfn = size_t(mesh->nfaces) * mesh->nfp;
-#define MG_MCASE(D, P)                                                                  \
-  if (mesh->dim == D && mesh->order == P) {                                             \
-    const size_t per_p = sizeof(double) * nfld * quad->nq;                              \
-    if (per_p > kBudget) return fail(MG_ERR_UNSUPPORTED, "quadrature too large for LDS"); \
-    int epb_p = int(std::max<size_t>(1, std::min<size_t>(8, 256 / quad->nq)));        \
-    ea.epb = epb_p;                                                                     \
-    auto kp = mgdg::esdg_project_mix_kernel<D, P>;                                      \
-    if ((s = set_lds(kp, kBudget))) return s;                                           \
-    hipLaunchKernelGGL(kp, dim3(unsigned((a.K + epb_p - 1) / epb_p)),                   \
-                       dim3(mgdg::kBlock), per_p * epb_p, st, a, ea);                  \
-    if ((s = check_launch("esdg_project_mix_kernel"))) return s;                        \
-    const size_t nchunk = (size_t(esdg->nh) + quad->nq - 1) / quad->nq;               \
-    const size_t nacc = nchunk * quad->nq + nft;                                        \
-    const size_t per_e = sizeof(mgdg::RnPair<D>) * esdg->nh +                           \
-        sizeof(double) * (nfld * (2 * size_t(mesh->np) + nfn + nft + nacc) +            \
-                          2 * size_t(mesh->np) + nfn + 2 * nft);                        \
-    if (per_e > kBudget) return fail(MG_ERR_UNSUPPORTED, "quadrature too large for LDS"); \
-    int epb = int(std::max<size_t>(1, std::min<size_t>(16, (64 * 1024) / per_e)));     \
-    ea.epb = epb;                                                                       \
-    auto kern = mgdg::esdg_mix_kernel<D, P>;                                            \
-    if ((s = set_lds(kern, kBudget))) return s;                                         \
-    hipLaunchKernelGGL(kern, dim3(unsigned((a.K + epb - 1) / epb)), dim3(mgdg::kBlock), \
-                       per_e * epb, st, a, ea);                                         \
-    return check_launch("esdg_mix_kernel");                                             \
-  }
+#define MG_MCASE(D, P) \
+  if (mesh->dim == D && mesh->order == P) return esdg_mix_launch<D, P>(a, ea, st);
   if (gas->nspecies != 7) return fail(MG_ERR_UNSUPPORTED, "the mixture has 7 species");
   MG_MCASE(2, 1) MG_MCASE(2, 2) MG_MCASE(2, 3) MG_MCASE(2, 4)
   MG_MCASE(3, 1) MG_MCASE(3, 2) MG_MCASE(3, 3)

@@ -2210,9 +2210,7 @@ struct EsdgArgs {
   int64_t nbq;
   double* ev;             // [F][N] projected entropy variables
   int dissipation;
-  // nq = 64, NF*nfq = 192, 256 threads: the paired phase 4 (each two-point
-  // flux once, for both rows) with the operators along cyclic diagonals
-  int paired;
+  // operators along cyclic diagonals (mg_esdg_pairs.h)
   const double* skew_diag;  // [DIM][nq(s)][nq(h)]: (Q_r - Q_r^T)[h][(h+s) % nq]
   const double* ext_diag;   // [nq(s)][NF*nfq(m)]: E[m][(m+s) % nq]
   // mixtures: Newton steps per point, exterior temperatures at the
@@ -2267,106 +2265,6 @@ __global__ __launch_bounds__(kBlock) void esdg_project_kernel(KArgs a, EsdgArgs 
     }
 #pragma unroll
     for (int f = 0; f < NFLD; ++f) ea.ev[f * N + e0 * NP + t] = v[f];
-  }
-}
-
-// Phase 4 of esdg_kernel when nq = 64 and NF*nfq = 192 (nh = 256, four
-// waves): each two-point flux is evaluated once.  (Q_h - Q_h^T) is skew and
-// F_S symmetric, so the pair (h, j) adds S[h][j] F_S to row h and the
-// negative to row j.  Wave 0 owns the 64 volume rows and meets the pairs
-// (h, (h+s) mod 64), s = 1..31, in step s; the contributions to the partner
-// rows travel in a register vector that moves one lane down per step, so
-// that lane h always holds row (h+s) mod 64 (s = 32 pairs each lane with the
-// lane that owns the same pair: both add their own row).  Wave 1 + b owns
-// face rows 64b..64b+63 and meets the volume points (l+s) mod 64 in step s,
-// s = 0..63 (the face-face block is zero); its moving vector collects that
-// block's part of the volume rows and is back in place after 64 steps.
-// Results: volume rows in the four nq-long pieces of s_acc (piece 0 from
-// wave 0, piece 1 + b from wave 1 + b; phase 5 adds them), face rows plus
-// the face flux in the face slots.  One element per workgroup: thread
-// 64 + m has computed face point m's flux (fkeep) in phase 3.
-template <int DIM, int NSP>
-__device__ __forceinline__ void esdg_pairs_64(const KArgs& a, const EsdgArgs& ea,
-                                              const EcPair<DIM, NSP>* s_prim,
-                                              const double (&fkeep)[2 + DIM + NSP],
-                                              double* s_acc, int64_t e, int nacc,
-                                              double gamma) {
-  constexpr int NF = DIM + 1;
-  constexpr int NFLD = 2 + DIM + NSP;
-  using Prim = EcPair<DIM, NSP>;
-  constexpr int NQ = 64, NFT = 192;
-  const int nfq = ea.nfq;
-  const int l = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int down = (l + 1) & 63;
-  {
-    const int le = 0, epb = 1;
-    const Prim* pj = s_prim;
-    double acc[NFLD], mv[NFLD];
-#pragma unroll
-    for (int f = 0; f < NFLD; ++f) acc[f] = mv[f] = 0.0;
-    if (wave == 0) {
-      const Prim ph = pj[l];
-      double rx[DIM * DIM];
-#pragma unroll
-      for (int k = 0; k < DIM * DIM; ++k) rx[k] = a.rx[e * DIM * DIM + k];
-      for (int s = 1; s <= 32; ++s) {
-        double sd[DIM];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) sd[d] = 0.0;
-#pragma unroll
-        for (int r = 0; r < DIM; ++r) {
-          const double sr = ea.skew_diag[(r * NQ + s) * NQ + l];
-#pragma unroll
-          for (int d = 0; d < DIM; ++d) sd[d] += rx[r * DIM + d] * sr;
-        }
-        double fv[NFLD];
-        ec_flux_dot<DIM, NSP, true>(ph, pj[(l + s) & 63], sd, gamma, fv);
-        if (s < 32) {
-#pragma unroll
-          for (int f = 0; f < NFLD; ++f) {
-            acc[f] += fv[f];
-            mv[f] = __shfl(mv[f] - fv[f], down, 64);
-          }
-        } else {
-#pragma unroll
-          for (int f = 0; f < NFLD; ++f) acc[f] += fv[f];
-        }
-      }
-      // lane l holds row (l + 32) mod 64
-#pragma unroll
-      for (int f = 0; f < NFLD; ++f) {
-        acc[f] += __shfl(mv[f], (l + 32) & 63, 64);
-        s_acc[(f * epb + le) * nacc + l] = acc[f];
-      }
-    } else {
-      const int m = (wave - 1) * NQ + l;
-      const Prim pm = pj[NQ + m];
-      const int fc = m / nfq;
-      const double bsc = a.fscale[e * NF + fc] * ea.wf[m - fc * nfq];
-      double nrm[DIM];
-#pragma unroll
-      for (int d = 0; d < DIM; ++d) nrm[d] = bsc * a.normals[(e * NF + fc) * DIM + d];
-      for (int s = 0; s < NQ; ++s) {
-        const double b = ea.ext_diag[s * NFT + m];
-        double sd[DIM];
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) sd[d] = b * nrm[d];
-        double fv[NFLD];
-        ec_flux_dot<DIM, NSP, true>(pm, pj[(l + s) & 63], sd, gamma, fv);
-#pragma unroll
-        for (int f = 0; f < NFLD; ++f) {
-          acc[f] -= fv[f];
-          mv[f] = __shfl(mv[f] + fv[f], down, 64);
-        }
-      }
-#pragma unroll
-      for (int f = 0; f < NFLD; ++f) {
-        double* row = s_acc + (f * epb + le) * nacc;
-        row[wave * NQ + l] = mv[f];
-        row[4 * NQ + m] = acc[f] + fkeep[f];
-      }
-    }
   }
 }
 
@@ -2584,7 +2482,7 @@ __global__ __launch_bounds__(kBlock) void esdg_kernel(KArgs a, EsdgArgs ea) {
   using E = Elem<DIM, P>;
   constexpr int NP = E::NP, NFP = E::NFP, NF = E::NF;
   constexpr int NFLD = 2 + DIM + NSP;
-  using Pair = EcPair<DIM, NSP>;
+  using Pair = EcPairLog<DIM, NSP>;
   extern __shared__ double lds[];
   const int nq = ea.nq, nfq = ea.nfq, nh = ea.nh, epb = ea.epb, nft = NF * ea.nfq;
   Pair* s_prim = reinterpret_cast<Pair*>(lds);             // [epb][nh]
@@ -2594,9 +2492,8 @@ __global__ __launch_bounds__(kBlock) void esdg_kernel(KArgs a, EsdgArgs ea) {
   // phase 4 splits volume rows into C pieces of nq entries
   const int C = (nh + nq - 1) / nq;
   const int nacc = C * nq + nft;                            // row sums per field
-  // face fluxes [F][epb][nft] (not in the paired layout: kept in registers)
-  double* s_fs = s_vp + NFLD * epb * NF * NFP;
-  double* s_qf = ea.paired ? s_fs : s_fs + NFLD * epb * nft;  // [F][epb][nft], 2-3
+  double* s_fs = s_vp + NFLD * epb * NF * NFP;              // [F][epb][nft]
+  double* s_qf = s_fs + NFLD * epb * nft;                   // [F][epb][nft], 2-3
   double* s_acc = s_qf;                                     // [F][epb][nacc], phases 4-5
   const int64_t e0 = int64_t(blockIdx.x) * epb;
   const int ne = a.K - e0 < epb ? int(a.K - e0) : epb;
@@ -2643,39 +2540,23 @@ __global__ __launch_bounds__(kBlock) void esdg_kernel(KArgs a, EsdgArgs ea) {
   }
   __syncthreads();
   // 3: entropy-stable face flux at the face points, times fscale * w
-  double fkeep[NFLD];
+  for (int t = threadIdx.x; t < ne * nft; t += blockDim.x) {
+    const int le = t / nft;
+    const int m = t - le * nft;
+    double fs[NFLD];
+    esdg_face_flux<DIM, P, NSP>(a, ea, s_qf, s_vp, s_q, e0, le, m, gamma, fs);
 #pragma unroll
-  for (int f = 0; f < NFLD; ++f) fkeep[f] = 0.0;
-  if (ea.paired) {
-    // one element per workgroup: thread 64 + m keeps face point m's flux
-    // for its face row in phase 4
-    const int m = int(threadIdx.x) - 64;
-    if (m >= 0 && m < nft && ne == 1)
-      esdg_face_flux<DIM, P, NSP>(a, ea, s_qf, s_vp, s_q, e0, 0, m, gamma, fkeep);
-  } else {
-    for (int t = threadIdx.x; t < ne * nft; t += blockDim.x) {
-      const int le = t / nft;
-      const int m = t - le * nft;
-      double fs[NFLD];
-      esdg_face_flux<DIM, P, NSP>(a, ea, s_qf, s_vp, s_q, e0, le, m, gamma, fs);
-#pragma unroll
-      for (int f = 0; f < NFLD; ++f) s_fs[(f * epb + le) * nft + m] = fs[f];
-    }
+    for (int f = 0; f < NFLD; ++f) s_fs[(f * epb + le) * nft + m] = fs[f];
   }
   __syncthreads();
   // 4: rows of (Q_h - Q_h^T) o F_S, plus the face flux on face rows.  A
   // volume row has nh entries, a face row nq (the face-face block is zero):
   // volume rows are cut into C = ceil(nh / nq) pieces of nq entries so that
   // every work item sums nq pairs; the pieces are added in phase 5.
-  if (ea.paired) {
-    esdg_pairs_64<DIM, NSP>(a, ea, s_prim, fkeep, s_acc, e0, nacc, gamma);
-  } else {
-    esdg_rows<DIM, NFLD>(a, ea, s_prim, s_fs, s_acc, e0, ne, nacc, C,
-                         [gamma](const Pair& x, const Pair& y, const double* sd,
-                                 double* acc) {
-                           ec_flux_dot<DIM, NSP>(x, y, sd, gamma, acc);
-                         });
-  }
+  esdg_rows<DIM, NFLD>(a, ea, s_prim, s_fs, s_acc, e0, ne, nacc, C,
+                       [gamma](const Pair& x, const Pair& y, const double* sd, double* acc) {
+                         ec_flux_dot<DIM, NSP>(x, y, sd, gamma, acc);
+                       });
   __syncthreads();
   // 5: dQ/dt = -M^-1 V_h^T acc
   esdg_apply<DIM, P, NFLD>(a, ea, s_acc, e0, ne, nacc, C);

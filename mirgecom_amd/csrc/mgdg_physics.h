@@ -34,6 +34,14 @@ struct GasDev {
   double ma_alpha, ma_factor, ma_epsilon, ma_singular;  // mixture-averaged
 };
 
+// a b + c with a wave-uniform c as the instruction's scalar operand (left to
+// the compiler, a Horner step copies it to two VGPRs first).
+__device__ __forceinline__ double fma_s(double a, double b, double c) {
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
+  return d;
+}
+
 // {{{ uiuc_7sp thermochemistry (species order C2H4, O2, CO2, CO, H2O, H2, N2)
 
 constexpr int MIX_NSP = 7;
@@ -70,6 +78,16 @@ struct PolyDev {
 // module); mg_load_mechanism / mg_load_transport fill every copy
 static __constant__ PolyDev c_poly;
 
+// The polynomials through a pointer the compiler cannot see through: their
+// scalar loads stay where the values are used.  Loops over points otherwise
+// have all of them hoisted, and hundreds of SGPRs spilled into VGPR lanes.
+using PolyConst = const __attribute__((address_space(4))) PolyDev;
+__device__ __forceinline__ PolyConst* poly_here() {
+  PolyConst* p = (PolyConst*)&c_poly;
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
 // Lowest and highest NASA7 switch temperature over the species: a wave whose
 // lanes all lie above the highest (below the lowest) needs only the high
 // (low) range, which the callers below evaluate alone in that case (the
@@ -90,6 +108,14 @@ __device__ __forceinline__ void nasa7_tmid_range(double& lo, double& hi) {
 // the range would turn every coefficient into a per-lane vector load).
 __device__ __forceinline__ double horner5(const double (&c)[5], double t) {
   return c[0] + t * (c[1] + t * (c[2] + t * (c[3] + t * c[4])));
+}
+
+template <typename C>
+__device__ __forceinline__ double horner5_s(const C& c, double t) {
+  double v = fma_s(t, c[4], c[3]);
+#pragma unroll
+  for (int i = 2; i >= 0; --i) v = fma_s(v, t, c[i]);
+  return v;
 }
 
 __device__ __forceinline__ void nasa7_cp_h(int k, double t, double inv_t, double& cp_r,
@@ -171,6 +197,74 @@ __device__ __forceinline__ double mix_temperature(double e_in, double t_seed,
     }
     t = t + (e_in - e) / cv;
   }
+  return t;
+}
+
+// Internal energy of mass fractions y as a polynomial in T for one NASA7
+// range: e(T) = c[5] + T (c[0] + c[1] T + ... + c[4] T^4), and the gas
+// constant r; c_v(T) = c[0] + 2 c[1] T + ... + 5 c[4] T^4.
+template <int RANGE>
+__device__ __forceinline__ void mix_e_poly(const double* y, double* c, double& r) {
+  PolyConst* poly = poly_here();
+  double s = 0.0;
+#pragma unroll
+  for (int i = 0; i < 6; ++i) c[i] = 0.0;
+#pragma unroll
+  for (int k = 0; k < MIX_NSP; ++k) {
+    const double w = c_mech.inv_wt[k] * y[k];
+    const auto* h = poly->h[RANGE][k];
+    s += w;
+#pragma unroll
+    for (int i = 0; i < 6; ++i) c[i] += w * h[i];
+  }
+#pragma unroll
+  for (int i = 0; i < 6; ++i) c[i] *= c_mech.gas_constant;
+  r = c_mech.gas_constant * s;
+  c[0] -= r;
+}
+
+// mix_temperature with the species summed into those polynomials once per
+// range instead of in every update; also c_v's coefficients cvp of the range
+// the result lies in (T_mid itself: the low one) and the gas constant.  A wave
+// whose lanes lie in both ranges updates by mix_e_cv.
+__device__ __forceinline__ double mix_temperature_poly(double e_in, double t_seed,
+                                                       const double* y, int niter,
+                                                       double* cvp, double& r) {
+  double tmid_lo, tmid_hi;
+  nasa7_tmid_range(tmid_lo, tmid_hi);
+  double t = t_seed, c[6], d[5];
+  int have = -1;
+  for (int it = 0; it <= niter; ++it) {
+    const int want = __all(t > tmid_hi) ? 1 : (__all(!(t > tmid_lo)) ? 0 : 2);
+    if (want != have && want != 2) {
+      if (want == 1)
+        mix_e_poly<1>(y, c, r);
+      else
+        mix_e_poly<0>(y, c, r);
+#pragma unroll
+      for (int i = 0; i < 5; ++i) d[i] = (i + 1) * c[i];
+      have = want;
+    }
+    if (want == 2) {
+      // both ranges; the result's own afterwards
+      if (it == niter) {
+        double ch[6];
+        mix_e_poly<1>(y, ch, r);
+        mix_e_poly<0>(y, c, r);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) d[i] = (i + 1) * (t > tmid_hi ? ch[i] : c[i]);
+      } else {
+        double e, cv;
+        mix_e_cv(t, y, e, cv);
+        t = t + (e_in - e) / cv;
+      }
+    } else if (it < niter) {
+      const double e = c[5] + t * (c[0] + t * (c[1] + t * (c[2] + t * (c[3] + t * c[4]))));
+      t = t + (e_in - e) / horner5(d, t);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 5; ++i) cvp[i] = d[i];
   return t;
 }
 
@@ -556,31 +650,34 @@ __device__ __forceinline__ void entropy_to_cons(const double* ev, double gamma,
   for (int k = 0; k < NSP; ++k) q[2 + DIM + k] = mass * (ev[2 + DIM + k] * gm1);
 }
 
-// Per-point quantities of the entropy-conserving flux, with the logarithms
-// of rho and beta = rho/(2p) taken once per point.
 template <int NSP>
 struct EcSpecies {
   double yh[NSP];  // Y / 2
 };
-// Without species one padding double makes a 3-D point 9 doubles: an odd
-// stride in 8-byte words, so that lanes reading consecutive points from LDS
-// spread over the banks (8 doubles put 64 lanes on 4 bank groups).
 template <>
-struct EcSpecies<0> {
-  double pad_;
+struct EcSpecies<0> {};
+
+// What the paired two-point flux reads of a point (kept in LDS per hybridized
+// point).  16-byte aligned for 16-byte LDS reads; in 3-D a point is 6 (14
+// with species) doubles, so that the 16 lanes of one read phase fall into
+// different banks.
+template <int DIM, int NSP>
+struct alignas(16) EcPair : EcSpecies<NSP> {
+  double rhoh;     // rho / 2
+  double beta;
+  double uh[DIM];  // u / 2
 };
 
-// What the two-point flux reads of a point (kept in LDS per hybridized point).
+// ... with rho, |u|^2 / 4 and the logarithms of rho and beta.
 template <int DIM, int NSP>
-struct EcPair : EcSpecies<NSP> {
-  double rho, lrho, beta, lbeta;
-  double kh;       // |u|^2 / 4
-  double uh[DIM];  // u / 2
+struct EcPairLog : EcPair<DIM, NSP> {
+  double rho, kh;
+  double lrho, lbeta;
 };
 
 // ... with the pressure and the wavespeed |u| + c the face flux needs.
 template <int DIM, int NSP>
-struct EcPrim : EcPair<DIM, NSP> {
+struct EcPrim : EcPairLog<DIM, NSP> {
   double p, c;
 };
 
@@ -588,6 +685,7 @@ template <int DIM, int NSP>
 __device__ __forceinline__ void ec_prim(const double* q, double gamma,
                                         EcPrim<DIM, NSP>& a) {
   a.rho = q[0];
+  a.rhoh = 0.5 * q[0];
   const double irho = 1.0 / q[0];
   double u2 = 0.0;
 #pragma unroll
@@ -635,13 +733,13 @@ __device__ __forceinline__ void ln_mean_parts(double x, double lx, double y, dou
 }
 
 // sum_d s_d F_S,d(a, b) of Chandrashekar's entropy-conserving, kinetic-
-// energy-preserving flux (mirgecom/inviscid.py:451-518), added to acc (SET:
-// stored into acc).  The energy flux needs 1 / ((gamma - 1) beta_mean): it
+// energy-preserving flux (mirgecom/inviscid.py:451-518), added to acc.  The
+// energy flux needs 1 / ((gamma - 1) beta_mean): it
 // is formed as den / num of beta's logarithmic mean; p_mean =
 // rho_avg / (2 beta_avg) = (rho_a + rho_b) / (2 (beta_a + beta_b)).
-template <int DIM, int NSP, bool SET = false>
-__device__ __forceinline__ void ec_flux_dot(const EcPair<DIM, NSP>& a,
-                                            const EcPair<DIM, NSP>& b,
+template <int DIM, int NSP>
+__device__ __forceinline__ void ec_flux_dot(const EcPairLog<DIM, NSP>& a,
+                                            const EcPairLog<DIM, NSP>& b,
                                             const double* s, double gamma,
                                             double* acc) {
   double rn, rd, bn, bd;
@@ -667,13 +765,134 @@ __device__ __forceinline__ void ec_flux_dot(const EcPair<DIM, NSP>& a,
   if constexpr (NSP > 0)
     for (int k = 0; k < NSP; ++k) v[2 + DIM + k] = mflux * (a.yh[k] + b.yh[k]);
 #pragma unroll
-  for (int f = 0; f < 2 + DIM + NSP; ++f) {
-    if constexpr (SET)
-      acc[f] = v[f];
-    else
-      acc[f] += v[f];
+  for (int f = 0; f < 2 + DIM + NSP; ++f) acc[f] += v[f];
+}
+
+// {{{ logarithmic means from their series (the paired pair loop)
+//
+// With z = (x - y) / (x + y) and f = z^2, ln x - ln y = 2 artanh z, so that
+//   ln-mean(x, y)     = (x + y) / 2 * P(f),  P = z / artanh z
+//   1 / ln-mean(x, y) = 2 / (x + y) * Q(f),  Q = artanh z / z = sum f^k / (2k + 1)
+// N + 1 terms leave a relative error below f^(N+1): 3e-18 for N = 3 at
+// f < 1e-4 (the reference's threshold) and 3e-17 for N = 9 at f < 3e-2.  The
+// loop takes the short series when all of a wave's pairs allow it (SHORT; the
+// mixture's pairs seldom do, and go to the long one at once), the long one
+// otherwise, and the logarithms themselves only in waves with a pair beyond
+// 3e-2 (values 42 % apart).
+constexpr double kLnNear = 1e-4, kLnFar = 3e-2;
+constexpr int kLnShort = 3, kLnLong = 9;
+
+struct LnSeries {
+  double p[kLnLong + 1], q[kLnLong + 1];
+};
+
+constexpr LnSeries make_ln_series() {
+  LnSeries s{};
+  for (int n = 0; n <= kLnLong; ++n) {
+    s.q[n] = 1.0 / (2 * n + 1);
+    double v = n == 0 ? 1.0 : 0.0;
+    for (int k = 1; k <= n; ++k) v -= s.q[k] * s.p[n - k];
+    s.p[n] = v;   // P Q = 1, term by term
+  }
+  return s;
+}
+
+template <int N>
+__device__ __forceinline__ void ln_pq(double f1, double f2, double& p, double& q) {
+  constexpr LnSeries c = make_ln_series();
+  p = fma_s(f1, c.p[N], c.p[N - 1]);
+  q = fma_s(f2, c.q[N], c.q[N - 1]);
+#pragma unroll
+  for (int k = N - 2; k >= 0; --k) {
+    p = fma_s(p, f1, c.p[k]);
+    q = fma_s(q, f2, c.q[k]);
   }
 }
+
+// Two quantities of a pair of points: sums s (x + y; of the first halves of
+// it) and differences d (x - y), is2 = 1 / s2, f the squared ratios; mean1 =
+// ln-mean of the first, inv2 = half the inverse ln-mean of the second.
+struct LnPair {
+  double s1, d1, s2, d2, is2, f1, f2;
+  double mean1, inv2;
+  __device__ __forceinline__ void begin() {
+    // 1/s1 and 1/s2 from one reciprocal
+    const double r = rcp_nr(s1 * s2);
+    is2 = r * s1;
+    const double z1 = d1 * (r * s2), z2 = d2 * is2;
+    f1 = z1 * z1;
+    f2 = z2 * z2;
+  }
+};
+
+// The means of R pairs at once (one branch, and the pairs' chains of
+// operations interleave); far(r, e1, e2) gives ln y - ln x of both
+// quantities of pair r.
+template <bool SHORT, int R, typename Far>
+__device__ __forceinline__ void ln_means(LnPair (&a)[R], Far far) {
+  double fm = 0.0, p[R], q[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) fm = fmax(fm, fmax(a[r].f1, a[r].f2));
+  bool all = SHORT && __all(fm < kLnNear);
+  if (all) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) ln_pq<kLnShort>(a[r].f1, a[r].f2, p[r], q[r]);
+  } else {
+#pragma unroll
+    for (int r = 0; r < R; ++r) ln_pq<kLnLong>(a[r].f1, a[r].f2, p[r], q[r]);
+    all = __all(fm < kLnFar);
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    a[r].mean1 = a[r].s1 * p[r];
+    a[r].inv2 = a[r].is2 * q[r];
+  }
+  if (!all) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      double e1, e2;
+      far(r, e1, e2);
+      if (!(a[r].f1 < kLnFar)) a[r].mean1 = -2.0 * a[r].d1 * rcp_nr(e1);
+      if (!(a[r].f2 < kLnFar)) a[r].inv2 = -0.5 * e2 * rcp_nr(a[r].d2);
+    }
+  }
+}
+
+// }}}
+
+// The direction-free parts of ec_flux_dot for the paired loop: the flux in
+// direction s is, with un = s . (u_a + u_b) / 2 and m = rho un,
+//   mass m, energy e m + p un, momentum m (u_a + u_b) / 2 + p s,
+// where e = 1 / (2 (gamma - 1) ln-mean(beta)) + u_a . u_b / 2 (the reference's
+// -(|u_a|^2 + |u_b|^2) / 4 + |u_a + u_b|^2 / 4).  begin() fills the pair's
+// logarithmic means' arguments, finish() takes the means.
+template <int DIM, int NSP_>
+struct EcPaired {
+  static constexpr int NSP = NSP_;
+  static constexpr int LOGS = 2;   // doubles between two points' logarithms
+  static constexpr int LOG2 = 1;   // ... and between a point's two
+  static constexpr bool SHORT = true;
+  static constexpr int NFLD = 2 + DIM + NSP;
+  using Point = EcPair<DIM, NSP>;
+  double inv_gm1;
+  __device__ __forceinline__ explicit EcPaired(double gamma) : inv_gm1(1.0 / (gamma - 1.0)) {}
+  __device__ __forceinline__ static void begin(const Point& a, const Point& b, LnPair& l) {
+    l.s1 = a.rhoh + b.rhoh;
+    l.d1 = a.rhoh - b.rhoh;
+    l.s2 = a.beta + b.beta;
+    l.d2 = a.beta - b.beta;
+    l.begin();
+  }
+  __device__ __forceinline__ void finish(const Point& a, const Point& b, const LnPair& l,
+                                         double& rho, double& e, double& p) const {
+    rho = l.mean1;
+    p = l.s1 * l.is2;
+    double uu = 0.0;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) uu += a.uh[d] * b.uh[d];
+    e = fma(2.0, uu, l.inv2 * inv_gm1);
+  }
+};
 
 // {{{ Renac's two-point flux (mixtures)
 
@@ -681,17 +900,18 @@ __device__ __forceinline__ void ec_flux_dot(const EcPair<DIM, NSP>& a,
 // NASA7 range when every active lane of the wave lies in it.
 template <int RANGE>
 __device__ __forceinline__ double mix_cv_range(double t, const double* y) {
+  PolyConst* poly = poly_here();
   double sc = 0.0;
 #pragma unroll
   for (int k = 0; k < MIX_NSP; ++k) {
     double cp;
     if constexpr (RANGE < 0) {
       const bool high = t > c_mech.t_mid[k];
-      const double cp_lo = horner5(c_poly.cp[0][k], t);
-      const double cp_hi = horner5(c_poly.cp[1][k], t);
+      const double cp_lo = horner5_s(poly->cp[0][k], t);
+      const double cp_hi = horner5_s(poly->cp[1][k], t);
       cp = high ? cp_hi : cp_lo;
     } else {
-      cp = horner5(c_poly.cp[RANGE][k], t);
+      cp = horner5_s(poly->cp[RANGE][k], t);
     }
     sc += c_mech.inv_wt[k] * (cp - 1.0) * y[k];
   }
@@ -734,6 +954,20 @@ struct RnPair {
   double rho, lrho, th, lth, pth, t;
   double uh[DIM];
   double yh[MIX_NSP];
+};
+
+// ... in the paired loop: with half of the point's part of the mixture c_v as
+// a polynomial in T (the NASA7 range the point lies in).  22 doubles in 3-D:
+// 4 mod 8 dwords, as EcPair.
+template <int DIM>
+struct alignas(16) RnPoint {
+  double rhoh, th;    // rho / 2, 1 / T
+  double pth, t;      // p / (2 T), T / 2
+  double uh[DIM];
+  double lrho[4 - DIM];   // ([0]; with lth read for far states only)
+  alignas(16) double yh[MIX_NSP];
+  double lth;
+  alignas(16) double cv[5];
 };
 
 // ... with the wavespeed |u| + c the face flux needs.
@@ -793,6 +1027,49 @@ __device__ __forceinline__ void rn_flux_dot(const RnPair<DIM>& a, const RnPair<D
 #pragma unroll
   for (int k = 0; k < MIX_NSP; ++k) acc[2 + DIM + k] += mflux * y[k];
 }
+
+// rn_flux_dot for the paired loop (see EcPaired; e = c_v(T_mean) T_mean +
+// u_a . u_b / 2).  POLY: every point of the element lies in one NASA7 range,
+// and so does T_mean, which lies between the two temperatures: c_v comes from
+// the points' polynomials.
+template <int DIM, bool POLY>
+struct RnPaired {
+  static constexpr int NSP = MIX_NSP;
+  static constexpr int LOGS = sizeof(RnPoint<DIM>) / sizeof(double);
+  static constexpr int LOG2 = MIX_NSP + 1;
+  static constexpr bool SHORT = false;
+  static constexpr int NFLD = 2 + DIM + NSP;
+  using Point = RnPoint<DIM>;
+  __device__ __forceinline__ static void begin(const Point& a, const Point& b, LnPair& l) {
+    l.s1 = a.rhoh + b.rhoh;
+    l.d1 = a.rhoh - b.rhoh;
+    l.s2 = a.th + b.th;
+    l.d2 = a.th - b.th;
+    l.begin();
+  }
+  __device__ __forceinline__ void finish(const Point& a, const Point& b, const LnPair& l,
+                                         double& rho, double& e, double& p) const {
+    rho = l.mean1;
+    const double t_mean = 2.0 * l.inv2;
+    p = (a.pth + b.pth) * (a.t + b.t);
+    double uu = 0.0;
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) uu += a.uh[d] * b.uh[d];
+    double cvm;
+    if constexpr (POLY) {
+      double c[5];
+#pragma unroll
+      for (int i = 0; i < 5; ++i) c[i] = a.cv[i] + b.cv[i];
+      cvm = horner5(c, t_mean);
+    } else {
+      double y[MIX_NSP];
+#pragma unroll
+      for (int k = 0; k < MIX_NSP; ++k) y[k] = a.yh[k] + b.yh[k];
+      cvm = mix_cv(t_mean, y);
+    }
+    e = fma(2.0, uu, cvm * t_mean);
+  }
+};
 
 // }}}
 
