@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <string>
 
+#include "mg_quad_ns_kernels.h"
 #include "mgdg_host.h"
 
 namespace {
@@ -34,12 +35,24 @@ mg_status quad_ns_check(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* q
 // LDS row strides = 4 mod 32 doubles (bank spread of the matrix-core reads)
 int bank_stride(int n) { return n + ((4 - n % 32) + 32) % 32; }
 
-// up to 80 KiB per workgroup (at least one element, at most 128 KiB)
+// Elements per workgroup: as many (at most 16) as leave room for two
+// workgroups on a CU (80 KiB each), at least one; one element may take up to
+// 128 KiB.
 constexpr size_t kQuadBudget = 128 * 1024;
 
-int quad_epb(size_t per_elem) {
-  int epb = int((80 * 1024) / per_elem);
-  return std::max(1, std::min(epb, 16));
+template <typename Kern, typename Lds>
+mg_status quad_launch(Kern kern, Lds lds, const char* name, const mgdg::KArgs& a,
+                      mgdg::QuadArgs& qa, hipStream_t st) {
+  auto bytes = [&](int epb) { return sizeof(double) * lds(qa.gs, qa.fs, epb); };
+  if (bytes(1) > kQuadBudget) return fail(MG_ERR_UNSUPPORTED, "quadrature too large for LDS");
+  int epb = 1;
+  while (epb < 16 && bytes(epb + 1) <= 80 * 1024) ++epb;
+  qa.epb = epb;
+  mg_status s = set_lds(kern, kQuadBudget);
+  if (s) return s;
+  hipLaunchKernelGGL(kern, dim3(unsigned((a.K + epb - 1) / epb)), dim3(mgdg::kBlock),
+                     bytes(epb), st, a, qa);
+  return check_launch(name);
 }
 
 void quad_args(mgdg::QuadArgs& qa, const mg_mesh* mesh, const mg_quad* quad,

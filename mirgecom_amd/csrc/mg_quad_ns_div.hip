@@ -14,14 +14,8 @@ mg_status mg_ns_rhs_quad(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* 
   if (!grad) return fail(MG_ERR_ARG, "grad NULL");
   if (flux_kind < 0 || flux_kind > 2) return fail(MG_ERR_ARG, "flux_kind");
   const int var = gas_variant(gas);
-  const int nfld = 2 + mesh->dim + gas->nspecies, nsd = (nfld + 1) * mesh->dim;
   const int gs = bank_stride(mesh->dim * quad->nq);
   const int fs = bank_stride(mesh->nfaces * quad->nfq);
-  const size_t nfn = size_t(mesh->nfaces) * mesh->nfp;
-  const size_t per_elem =
-      sizeof(double) * (size_t(nfld) * (mesh->np + gs + fs + nfn) +
-                        size_t(nsd) * (mesh->np + nfn) + (var != 0 ? mesh->np + nfn : 0));
-  if (per_elem > kQuadBudget) return fail(MG_ERR_UNSUPPORTED, "quadrature too large for LDS");
   mgdg::KArgs a = make_args(mesh, gas);
   a.q = q;
   a.grad = grad;
@@ -30,18 +24,14 @@ mg_status mg_ns_rhs_quad(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* 
   a.inviscid_on = inviscid_on ? 1 : 0;
   mgdg::QuadArgs qa{};
   quad_args(qa, mesh, quad, temperature, q_bnd_quad, t_bnd_quad, niter);
-  qa.epb = quad_epb(per_elem);
   qa.gs = gs;
   qa.fs = fs;
-  const size_t lds = per_elem * qa.epb;
-  const unsigned nblk = unsigned((a.K + qa.epb - 1) / qa.epb);
   hipStream_t st = static_cast<hipStream_t>(stream);
 #define MG_DCASE(D, P, NS, MX)                                                      \
   if (mesh->dim == D && mesh->order == P && gas->nspecies == NS && var == MX) {     \
-    auto kern = mgdg::ns_div_quad_kernel<D, P, NS, MX>;                             \
-    if ((s = set_lds(kern, kQuadBudget))) return s;                                 \
-    hipLaunchKernelGGL(kern, dim3(nblk), dim3(mgdg::kBlock), lds, st, a, qa);       \
-    return check_launch("ns_div_quad_kernel");                                      \
+    return quad_launch(mgdg::ns_div_quad_kernel<D, P, NS, MX>,                      \
+                       mgdg::quad_div_lds<D, P, NS, MX>, "ns_div_quad_kernel", a,   \
+                       qa, st);                                                     \
   }
   MG_NSQ_CASES(MG_DCASE)
 #undef MG_DCASE
