@@ -8,7 +8,7 @@
 //
 // Network layout (all widths padded to the matrix-core tiles):
 //   input  32 features: (log T, log p, Y_1..Y_7, dt) normalised, then zeros
-//   hidden 256, 256, 256 with GELU (erf form)
+//   hidden 256, 256, 256 with GELU (tanh form)
 //   output 32: normalised dY_k over the substep dt in 0..6, zeros after
 // Parameters: one FP32 master array (W_l as [K_in][N_out] row-major, then
 // b_l, layer by layer; MG_MLP_NPARAM values) and BF16 copies of every W_l

@@ -34,12 +34,14 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 // GELU in its tanh form (Hendrycks & Gimpel 2016, eq. for the fast
 // approximation): gelu(z) = z (1 + tanh u) / 2, u = sqrt(2/pi) (z + 0.044715 z^3).
 // With E = exp(2u) and r = 1 / (1 + E): tanh u = 1 - 2r, so
-//   gelu(z)  = z (1 - r)
+//   gelu(z)  = z (1 - r) = z / (1 + exp(-2u))
 //   gelu'(z) = (1 - r) + 2 z r (1 - r) sqrt(2/pi) (1 + 3 * 0.044715 z^2)
 // evaluated with the hardware exp2 and reciprocal (v_exp_f32, v_rcp_f32),
 // about 1e-7 relative: far below the BF16 rounding of the activations.  The
 // erf form costs several times the VALU work and, at 128 activations per
 // lane and layer, outweighed the matrix-core time of the fused inference.
+// gelu takes 5 full-rate operations beside the two (all factors of the
+// exponent in two constants; z (1 - r) took 8 and cancelled for z < 0).
 constexpr float kGeluC0 = 0.7978845608028654f;   // sqrt(2 / pi)
 constexpr float kGeluC1 = 0.044715f;
 constexpr float kLog2e2 = 2.0f * 1.4426950408889634f;
@@ -49,7 +51,11 @@ __device__ __forceinline__ float gelu_r(float z) {
   const float e = __builtin_amdgcn_exp2f(kLog2e2 * u);
   return __builtin_amdgcn_rcpf(1.0f + e);
 }
-__device__ __forceinline__ float gelu(float z) { return z * (1.0f - gelu_r(z)); }
+__device__ __forceinline__ float gelu(float z) {
+  constexpr float k0 = -kLog2e2 * kGeluC0, k1 = k0 * kGeluC1;
+  const float e = __builtin_amdgcn_exp2f(z * (z * z * k1 + k0));
+  return z * __builtin_amdgcn_rcpf(1.0f + e);
+}
 __device__ __forceinline__ float gelu_grad(float z) {
   const float r = gelu_r(z);
   return (1.0f - r) + 2.0f * z * r * (1.0f - r) * kGeluC0 * (1.0f + 3.0f * kGeluC1 * z * z);
@@ -275,11 +281,14 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(GemmArgs g) {
   const int64_t k_lo = int64_t(blockIdx.z) * kper;
   const int r = lane & 15, kq = (lane >> 4) * 8;
   floatx4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
   const bool ncol1 = n0 + 16 < g.n;   // second column fragment exists
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    float b = 0.0f;   // z from its bias, in the order of the fused inference
+    if (EPI == kEpiGelu && n0 < g.n && (j == 0 || ncol1)) b = g.bias[n0 + 16 * j + r];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) acc[i][j] = floatx4{b, b, b, b};
+  }
   if (n0 < g.n) {
     for (int64_t k0 = k_lo; k0 < k_lo + kper; k0 += 32) {
       bf16x8 fa[2], fb[2];
@@ -313,11 +322,10 @@ __global__ __launch_bounds__(256) void gemm_nt_kernel(GemmArgs g) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) c[(row0 + e) * g.ldc + col] = acc[i][j][e] + b;
       } else if constexpr (EPI == kEpiGelu) {
-        const float b = g.bias[col];
         bf16x4 t;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float z = acc[i][j][e] + b;
+          const float z = acc[i][j][e];
           g.zout[(row0 + e) * g.n + col] = z;
           const __bf16 h = __bf16(gelu(z));
           g.out[(row0 + e) * g.n + col] = h;
@@ -467,11 +475,45 @@ static __global__ __launch_bounds__(256) void adam_kernel(float* __restrict__ pr
 // = sample_offset mod sample_period) whose surrogate source misses the exact
 // one by more than check_tol output scales, sends the whole element to the
 // exact rates (mix_species_source).
+//
+// Bound by the vector units (GELU is 60 % of their instructions) and the matrix
+// cores after each other: the first are busy 64 %, the second 27 % of the
+// time.  1.97 M nodes, np = 10: 1282 us with an 8-operation GELU, the bias
+// added behind it and the sampled check at the end; 1116 us with GELU in 5,
+// the sums started from the bias and the check moved beside the features;
+// 1080 us with every layer's first weights fetched before its barrier.  Raised
+// wave priorities for the products (1084-1092 us) do not overlap the two any
+// better.
 
 constexpr int kRows = 128;
 constexpr int kLdsStride = kH + 8;
 constexpr int kOutStride = kLdsStride / 2;   // output rows over activation rows (floats)
 static_assert(kOut <= kOutStride, "an output row fits an activation row");
+
+// The first weight fragments and the biases of a layer, fetched before the
+// barrier that ends the layer before it.
+struct LayerHead {
+  bf16x8 fw[4];
+  floatx4 b[4];
+};
+template <int KDIM>
+__device__ __forceinline__ void load_weights(bf16x8* fw, const __bf16* __restrict__ wt, int k0,
+                                             int w, int lane) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    fw[j] = *reinterpret_cast<const bf16x8*>(
+        wt + int64_t(w * 64 + 16 * j + (lane & 15)) * KDIM + k0 + (lane >> 4) * 8);
+}
+template <int KDIM>
+__device__ __forceinline__ void load_head(LayerHead& h, const __bf16* __restrict__ wt,
+                                          const float* __restrict__ bias, int w, int lane) {
+  load_weights<KDIM>(h.fw, wt, 0, w, lane);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float* b = bias + w * 64 + 16 * j + 4 * (lane >> 4);
+    h.b[j] = floatx4{b[0], b[1], b[2], b[3]};
+  }
+}
 
 // One hidden layer of the fused inference, in place on the activations
 // act [128][kLdsStride] (BF16, LDS), formed transposed: D = W X^T with the
@@ -481,25 +523,19 @@ static_assert(kOut <= kOutStride, "an output row fits an activation row");
 // conversion.  Wave w owns output features [64 w, 64 w + 64) of every row:
 // 4 x 8 accumulator fragments; the weight fragments of the next K step are
 // fetched while the current one's 32 matrix-core products run (two register
-// sets).
-template <int KDIM>
+// sets), the next layer's first ones (next) before the closing barrier.  The
+// sums start from the bias, which the GELU loop then need not add.
+template <int KDIM, typename Next>
 __device__ __forceinline__ void hidden_layer(__bf16* act, const __bf16* __restrict__ wt,
-                                             const float* __restrict__ bias, int w,
-                                             int lane) {
+                                             LayerHead& h, int w, int lane, Next next) {
   constexpr int NKS = KDIM / 32;
   const int r16 = lane & 15, kq = (lane >> 4) * 8;
   const int c0 = w * 64;
-  floatx4 acc[4][8];   // [out tile j][row tile i]: D[out][row]
+  floatx4 acc[4][8];   // [out tile j][row tile i]: D[out][row], from the bias
 #pragma unroll
   for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[j][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-  auto load_w = [&](bf16x8* fw, int k0) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      fw[j] = *reinterpret_cast<const bf16x8*>(wt + int64_t(c0 + 16 * j + r16) * KDIM + k0 +
-                                               kq);
-  };
+    for (int i = 0; i < 8; ++i) acc[j][i] = h.b[j];
   auto mma = [&](const bf16x8* fw, int k0) {
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -510,16 +546,15 @@ __device__ __forceinline__ void hidden_layer(__bf16* act, const __bf16* __restri
         acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw[j], fx, acc[j][i], 0, 0, 0);
     }
   };
-  bf16x8 fw0[4], fw1[4];
-  load_w(fw0, 0);
   if constexpr (NKS == 1) {
-    mma(fw0, 0);
+    mma(h.fw, 0);
   } else {
+    bf16x8 fw1[4];
 #pragma unroll 1
     for (int ks = 0; ks < NKS; ks += 2) {
-      load_w(fw1, (ks + 1) * 32);
-      mma(fw0, ks * 32);
-      if (ks + 2 < NKS) load_w(fw0, (ks + 2) * 32);
+      load_weights<KDIM>(fw1, wt, (ks + 1) * 32, w, lane);
+      mma(h.fw, ks * 32);
+      if (ks + 2 < NKS) load_weights<KDIM>(h.fw, wt, (ks + 2) * 32, w, lane);
       mma(fw1, (ks + 1) * 32);
     }
   }
@@ -527,18 +562,16 @@ __device__ __forceinline__ void hidden_layer(__bf16* act, const __bf16* __restri
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int o = c0 + 16 * j + 4 * (lane >> 4);   // this lane's 4 output features
-    float b[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) b[e] = bias[o + e];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       floatx4 v;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = gelu(acc[j][i][e] + b[e]);
+      for (int e = 0; e < 4; ++e) v[e] = gelu(acc[j][i][e]);
       *reinterpret_cast<bf16x4*>(act + (16 * i + r16) * kLdsStride + o) =
           __builtin_convertvector(v, bf16x4);
     }
   }
+  next();
   __syncthreads();
 }
 
@@ -564,6 +597,11 @@ struct InferArgsT {
 using InferArgs = InferArgsT<0>;
 static_assert(sizeof(InferArgsT<0>) == sizeof(InferArgsT<1>), "argument block layouts");
 
+// nodes whose surrogate source is checked against the exact rates
+__device__ __forceinline__ bool sampled(const Norm& nm, int64_t g) {
+  return nm.sample_period > 0 && g % nm.sample_period == nm.sample_offset;
+}
+
 template <typename A>
 __device__ __forceinline__ void infer_body(const A& a, int64_t blk) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -572,7 +610,8 @@ __device__ __forceinline__ void infer_body(const A& a, int64_t blk) {
   // of activation row r (each wave reads and writes only its own 32 rows
   // there), so that two workgroups fit a CU's LDS
   float* outp = reinterpret_cast<float*>(smem_raw);                    // [128][132]
-  int* eflag = reinterpret_cast<int*>(act + kRows * kLdsStride);       // [128]
+  double* s_ex = reinterpret_cast<double*>(act + kRows * kLdsStride);  // [7][128]
+  int* eflag = reinterpret_cast<int*>(s_ex + MIX_NSP * kRows);         // [128]
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
   const int epb = kRows / a.np;
@@ -581,7 +620,14 @@ __device__ __forceinline__ void infer_body(const A& a, int64_t blk) {
   const int64_t n = a.n;
   const int sp0 = 2 + a.dim;
 
-  // input features; out-of-bounds nodes flag their element
+  // generic views of the weights (the compiler keeps the global address
+  // space the argument block states)
+  const __bf16* wbf = (const __bf16*)a.wbf;
+  const float* prm = (const float*)a.prm;
+  // input features; out-of-bounds nodes flag their element.  Meanwhile the
+  // other two waves evaluate the sampled nodes' exact rates (one or two lanes
+  // of 128, as long as the features: 7,700 of a workgroup's 77,000 cycles
+  // when the waves with the features evaluated them at the end)
   if (threadIdx.x < kRows) eflag[threadIdx.x] = 0;
   __syncthreads();
   if (threadIdx.x < kRows) {
@@ -607,41 +653,56 @@ __device__ __forceinline__ void infer_body(const A& a, int64_t blk) {
 #pragma unroll
     for (int f = 0; f < kIn; ++f) act[rr * kLdsStride + f] = __bf16(f < kNIn ? xf[f] : 0.0f);
     if (!ok) atomicOr(&eflag[rr / a.np], 1);
+  } else if (threadIdx.x < 2 * kRows) {
+    const int rr = threadIdx.x - kRows;
+    const int64_t g = node0 + rr;
+    if (rr < rows && g < n && sampled(a.nm, g)) {
+      const double rho = a.q[g];
+      double y[MIX_NSP], ex[MIX_NSP];
+#pragma unroll
+      for (int k = 0; k < MIX_NSP; ++k) y[k] = a.q[(sp0 + k) * n + g] / rho;
+      mgdg::mix_species_source(rho, a.temp[g], y, ex);
+#pragma unroll
+      for (int k = 0; k < MIX_NSP; ++k) s_ex[k * kRows + rr] = ex[k];
+    }
   }
-  __syncthreads();
-
   const int r16 = lane & 15, kq = (lane >> 4) * 8;
   // hidden layers
-  // generic views of the weights (the compiler keeps the global address
-  // space the argument block states)
-  const __bf16* wbf = (const __bf16*)a.wbf;
-  const float* prm = (const float*)a.prm;
-  hidden_layer<kIn>(act, wbf + kBfW1, prm + kOffB1, w, lane);
-  hidden_layer<kH>(act, wbf + kBfW2, prm + kOffB2, w, lane);
-  hidden_layer<kH>(act, wbf + kBfW3, prm + kOffB3, w, lane);
+  LayerHead head;
+  load_head<kIn>(head, wbf + kBfW1, prm + kOffB1, w, lane);
+  __syncthreads();
+  hidden_layer<kIn>(act, wbf + kBfW1, head, w, lane,
+                    [&] { load_head<kH>(head, wbf + kBfW2, prm + kOffB2, w, lane); });
+  hidden_layer<kH>(act, wbf + kBfW2, head, w, lane,
+                   [&] { load_head<kH>(head, wbf + kBfW3, prm + kOffB3, w, lane); });
+  bf16x8 fo[kH / 32][2];
+  hidden_layer<kH>(act, wbf + kBfW3, head, w, lane, [&] {
+#pragma unroll
+    for (int ks = 0; ks < kH / 32; ++ks)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        fo[ks][j] = *reinterpret_cast<const bf16x8*>(wbf + kBfW4 +
+                                                     int64_t(16 * j + r16) * kH + 32 * ks + kq);
+  });
   // output layer (32 columns: 2 fragments): wave w owns row fragments
   // 2w, 2w + 1
   {
-    const __bf16* wt = wbf + kBfW4;
     const float* bias = prm + kOffB4;
     floatx4 acc[2][2];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (int k0 = 0; k0 < kH; k0 += 32) {
-      bf16x8 fb[2];
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-        fb[j] = *reinterpret_cast<const bf16x8*>(wt + int64_t(16 * j + r16) * kH + k0 + kq);
+    for (int k0 = 0; k0 < kH; k0 += 32) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
         const bf16x8 fa = *reinterpret_cast<const bf16x8*>(
             act + (16 * (2 * w + i) + r16) * kLdsStride + k0 + kq);
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fb[j], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa, fo[k0 / 32][j], acc[i][j],
+                                                              0, 0, 0);
       }
     }
 #pragma unroll
@@ -673,13 +734,11 @@ __device__ __forceinline__ void infer_body(const A& a, int64_t blk) {
     for (int k = 0; k < MIX_NSP; ++k)
       src[k] = (double(outp[rr * kOutStride + k]) * a.nm.out_scale[k] + a.nm.out_mean[k]) *
                irdt;
-    if (a.nm.sample_period > 0 && g % a.nm.sample_period == a.nm.sample_offset) {
-      double ex[MIX_NSP];
-      mgdg::mix_species_source(rho, a.temp[g], y, ex);
+    if (sampled(a.nm, g)) {
       bool bad = false;
 #pragma unroll
       for (int k = 0; k < MIX_NSP; ++k)
-        bad = bad || !(fabs(src[k] - ex[k]) <= a.nm.check_tol * a.nm.out_scale[k] * irdt);
+        bad = bad || !(fabs(src[k] - s_ex[k * kRows + rr]) <= a.nm.check_tol * a.nm.out_scale[k] * irdt);
       if (bad) atomicOr(&eflag[rr / a.np], 1);
     }
   }
@@ -708,7 +767,8 @@ static __global__ __launch_bounds__(256, 2) void infer_kernel(InferArgs a) {
 }
 
 // LDS bytes of infer_body / infer_kernel
-constexpr size_t kInferLds = sizeof(__bf16) * kRows * kLdsStride + sizeof(int) * kRows;
+constexpr size_t kInferLds = sizeof(__bf16) * kRows * kLdsStride +
+                             (sizeof(double) * MIX_NSP + sizeof(int)) * kRows;
 
 // }}}
 
