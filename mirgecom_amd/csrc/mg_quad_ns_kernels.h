@@ -1,6 +1,8 @@
 // Kernels of the overintegrated Navier-Stokes operator (ns_operator with a
 // quadrature tag).
 #pragma once
+#include <type_traits>
+
 #include "mgdg_kernels.h"
 
 namespace mgdg {
@@ -23,29 +25,43 @@ namespace mgdg {
 //
 // A workgroup owns epb elements.  LDS: s_n the nodal values, node by node
 // [epb][NP + NF NFP][ST] -- the element's nodes, then the neighbours' values at
-// its face nodes (interior faces); columns q, T (mixtures), and from the even
-// column G0 the gradients (divergence) -- then the point values: s_g
-// [cols][gs], s_f [cols][fs], row strides 4 mod 32 doubles for the matrix
-// cores' operand reads, and the results s_o.
+// its face nodes (interior faces); columns q, T (mixtures), and from column G0
+// the gradients (divergence) without the energy's, which no flux takes -- then
+// the point values: s_g [cols][gs], s_f [cols][fs], row strides 4 mod 32
+// doubles for the matrix cores' operand reads, and the results s_o.
 //
 // The points are dealt to the waves 64 at a time, volume points first, so that
-// the waves' shares differ by at most one such task.  Interpolations read a
-// node's columns with 16-byte LDS broadcasts, several nodes per step, the
-// next step's weights and face nodes already on their way.  (Node by node
-// each waited for its weight, then for the face node's index, then for LDS,
-// and one wave could hold three tasks while another held one: 73,000 of a
-// workgroup's 102,000 cycles at p = 3, ideal gas.)  ST is
-// 2 mod 4 doubles, which spreads the node-by-node writes over the LDS banks.
+// the waves' shares differ by at most one such task.  In 3-D the interpolations
+// to them are matrix products of the nodal columns with the points' weights.
+// Read by every lane instead, a node's columns are 16-byte LDS broadcasts of
+// two columns each: at the matrix cores' rate, one wave's keep LDS busy for as
+// long as its products take, and the four SIMDs share it.  Ideal gas, p = 3,
+// 82,944 elements, 64 volume and 48 face points: divergence 2194 -> 1317 us;
+// mixture, p = 2, 24,576 elements: 1057 -> 1000 us.  (The gradient, 5 columns,
+// stays at 880 us: its contraction takes as long as its points.)  2-D faces
+// have p + 1 points, which would leave most of a tile empty: there the lanes
+// keep reading the columns, several nodes per step, the next step's weights and
+// face nodes already on their way.  ST is 2 mod 4 doubles, which spreads the
+// node-by-node writes over the LDS banks.
 template <int DIM, int P, int NSP, int MIX, bool GRAD>
 struct QuadNs {
   using E = Elem<DIM, P>;
+  static constexpr bool MM = DIM == 3;   // interpolation on the matrix cores
   static constexpr int NFLD = 2 + DIM + NSP, NS = NFLD + 1, NSD = NS * DIM;
   static constexpr int NQC = NFLD + (MIX != 0 ? 1 : 0);
-  static constexpr int G0 = (NQC + 1) / 2 * 2;
-  static constexpr int NCOL = GRAD ? G0 + NSD : NQC;
+  static constexpr int NG = NSD - DIM;   // the viscous flux takes no energy gradient
+  static constexpr int G0 = MM ? NQC : (NQC + 1) / 2 * 2;
+  static constexpr int NCOL = GRAD ? G0 + NG : NQC;
+  static constexpr int NC4 = (NCOL + 3) / 4 * 4;
+  // columns interpolated together before the point's state is formed
+  static constexpr int NC1 = NC4 > 20 ? 16 : NC4;
   static constexpr int ST = (NCOL + 1) / 4 * 4 + 2;
+  // columns past NCOL up to NC4 (never used) are the next row's, or, behind the
+  // last row, these
+  static constexpr int PAD = MM ? 4 : 0;
   static constexpr int ROWS = E::NP + E::NFN;
-  static_assert(ST >= NCOL && ST % 4 == 2, "LDS row stride");
+  static_assert(ST >= NCOL && ST % 4 == 2 && (!MM || NC4 - ST <= PAD), "LDS row stride");
+  static_assert(NQC <= NC1 || !MM, "the state's columns");
 };
 
 // The contraction's K range is cut over ks waves per tile while that keeps
@@ -62,7 +78,7 @@ template <int DIM, int P, int NSP, int MIX>
 constexpr size_t quad_div_lds(int gs, int fs, int epb) {
   using C = QuadNs<DIM, P, NSP, MIX, true>;
   using E = Elem<DIM, P>;
-  const size_t nodes = size_t(epb) * C::ROWS * C::ST;
+  const size_t nodes = size_t(epb) * C::ROWS * C::ST + C::PAD;
   const size_t parts = size_t(quad_ksplit(quad_tiles(E::NP, C::NFLD * epb))) * C::NFLD * epb *
                        E::NP;
   // (the results go over the nodal values)
@@ -72,7 +88,7 @@ template <int DIM, int P, int NSP, int MIX>
 constexpr size_t quad_grad_lds(int gs, int fs, int epb) {
   using C = QuadNs<DIM, P, NSP, MIX, false>;
   using E = Elem<DIM, P>;
-  const size_t nodes = size_t(epb) * C::ROWS * C::ST;
+  const size_t nodes = size_t(epb) * C::ROWS * C::ST + C::PAD;
   const size_t out = size_t(C::NSD) * epb * E::NP;
   return (nodes > out ? nodes : out) + size_t(C::NS) * epb * (gs + fs);
 }
@@ -101,13 +117,13 @@ __device__ __forceinline__ void quad_load_nodes(const KArgs& a, const QuadArgs& 
     if constexpr (MIX != 0) v[C::NFLD] = qa.temp[g];
     if constexpr (GRAD) {
 #pragma unroll
-      for (int k = 0; k < C::NSD; ++k) v[C::G0 + k] = a.grad[k * N + g];
+      for (int k = 0; k < C::NG; ++k) v[C::G0 + k] = a.grad[(k < DIM ? k : k + DIM) * N + g];
     }
 #pragma unroll
     for (int f = 0; f < C::NQC; ++f) row[f] = v[f];
     if constexpr (GRAD) {
 #pragma unroll
-      for (int k = 0; k < C::NSD; ++k) row[C::G0 + k] = v[C::G0 + k];
+      for (int k = 0; k < C::NG; ++k) row[C::G0 + k] = v[C::G0 + k];
     }
   }
 }
@@ -156,6 +172,207 @@ __device__ __forceinline__ void quad_interp(const double* w, int ws, const doubl
   }
 }
 
+// {{{ interpolation on the matrix cores
+//
+// A wave interpolates 4 tiles of 16 points: D[column][point] +=
+// A[column][node] B[node][point], 16 columns to a v_mfma_f64_16x16x4 and 4 to
+// each v_mfma_f64_4x4x4 (four blocks: 4 columns x 16 points), which have the
+// same operand and result lanes: lane (kk, li) = (lane / 16, lane % 16) holds
+// B of node kk and point li, A of node kk and column li (li % 4), and gets
+// columns 4 g + kk of point li.  Transposing the 4 x 4 (tile, kk) squares over
+// registers and rows of 16 lanes then gives every lane all columns of the one
+// point (lane / 16, li).
+
+// r[t] in lane row k -> r[k] in lane row t
+__device__ __forceinline__ void quad_transpose(double* r) {
+  unsigned v[4][2];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) __builtin_memcpy(v[t], &r[t], 8);
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const auto x = __builtin_amdgcn_permlane32_swap(v[t][h], v[t + 2][h], false, false);
+      v[t][h] = x[0];
+      v[t + 2][h] = x[1];
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t += 2) {
+      const auto x = __builtin_amdgcn_permlane16_swap(v[t][h], v[t + 1][h], false, false);
+      v[t][h] = x[0];
+      v[t + 1][h] = x[1];
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t) __builtin_memcpy(&r[t], v[t], 8);
+}
+
+// A wave's accumulators: NC columns (a multiple of 4) of 4 tiles.
+template <int NC>
+struct QuadAcc {
+  static constexpr int NB = NC / 16, NQ = NC % 16 / 4;
+  doublex4 b[4][NB > 0 ? NB : 1];
+  double q[4][NQ > 0 ? NQ : 1];
+
+  __device__ __forceinline__ void zero() {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) b[t][i] = doublex4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int i = 0; i < NQ; ++i) q[t][i] = 0.0;
+    }
+  }
+  // one step of 4 nodes of tile t: this lane's node row and its weight
+  __device__ __forceinline__ void step(int t, const double* row, double w) {
+    const int li = threadIdx.x & 15;
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      b[t][i] = __builtin_amdgcn_mfma_f64_16x16x4f64(row[16 * i + li], w, b[t][i], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < NQ; ++i)
+      q[t][i] = __builtin_amdgcn_mfma_f64_4x4x4f64(row[16 * NB + 4 * i + (li & 3)], w,
+                                                   q[t][i], 0, 0, 0);
+  }
+  __device__ __forceinline__ void points(double* out) {
+#pragma unroll
+    for (int i = 0; i < NC / 4; ++i) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) out[4 * i + t] = i < 4 * NB ? b[t][i / 4][i % 4] : q[t][i - 4 * NB];
+      quad_transpose(out + 4 * i);
+    }
+  }
+};
+
+// The 4 tiles of a wave, and this lane's point among them.  Tiles beyond the
+// last and points beyond a tile's n repeat the last one (valid = false).
+template <int DIM, int P>
+struct QuadTiles {
+  using E = Elem<DIM, P>;
+  bool valid;
+  int le, fc, m;   // this lane's point
+  int m0;          // its tile's first point
+
+  QuadTiles() = default;
+  __device__ __forceinline__ QuadTiles(bool face, int task, int ne, int n) {
+    const int lane = threadIdx.x & 63;
+    const int per = (n + 15) / 16, nt = ne * per * (face ? E::NF : 1);
+    const int u = task * 4 + (lane >> 4), t = u < nt ? u : nt - 1;
+    const int r = t / per;
+    m0 = (t - r * per) * 16;
+    le = face ? r / E::NF : r;
+    fc = face ? r - le * E::NF : 0;
+    const int k = m0 + (lane & 15);
+    valid = u < nt && k < n;
+    m = k < n ? k : n - 1;
+  }
+  // this lane's point column of tile t's weights (n points to a node)
+  __device__ __forceinline__ int column(int t, int n) const {
+    const int k = __builtin_amdgcn_readlane(m0, 16 * t) + int(threadIdx.x & 15);
+    return k < n ? k : n - 1;
+  }
+};
+
+// Columns [C0, C0 + NC) at volume points; s_n: node rows of stride ST,
+// rows node rows to an element.
+template <int DIM, int P, int C0, int NC, int ST, int ROWS>
+__device__ __forceinline__ void quad_mm_volume(const double* interp, int nq,
+                                               const QuadTiles<DIM, P>& tl, const double* s_n,
+                                               double* out) {
+  constexpr int NP = Elem<DIM, P>::NP, NK = (NP + 3) / 4;
+  const int kk = (threadIdx.x >> 4) & 3;
+  int col[4], row[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    col[t] = tl.column(t, nq);
+    row[t] = __builtin_amdgcn_readlane(tl.le, 16 * t) * ROWS * ST + C0;
+  }
+  QuadAcc<NC> acc;
+  acc.zero();
+  double wn[4];
+  auto weights = [&](int s) {
+    const int k = 4 * s + kk;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const double w = interp[(k < NP ? k : NP - 1) * nq + col[t]];
+      wn[t] = k < NP ? w : 0.0;
+    }
+  };
+  weights(0);
+#pragma unroll 1
+  for (int s = 0; s < NK; ++s) {
+    double w[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) w[t] = wn[t];
+    weights(s + 1 < NK ? s + 1 : 0);
+    const int k = 4 * s + kk < NP ? 4 * s + kk : NP - 1;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc.step(t, s_n + row[t] + k * ST, w[t]);
+  }
+  acc.points(out);
+}
+
+// Face points: the weights and both sides' node rows, shared by the two sides'
+// (and all columns') interpolations.
+template <int DIM, int P, int ST, int ROWS>
+struct QuadFaceTiles {
+  using E = Elem<DIM, P>;
+  static constexpr int NFP = E::NFP, NK = (NFP + 3) / 4;
+  double w[NK][4];
+  int own[NK][4], ext[4];
+
+  QuadFaceTiles() = default;
+  // v0: the face's first exterior map entry of this lane's point (boundary
+  // faces, v0 < 0: the exterior rows are the own ones)
+  __device__ __forceinline__ QuadFaceTiles(const double* finterp, int nfq,
+                                           const QuadTiles<DIM, P>& tl, const int* s_fm,
+                                           int32_t v0) {
+    const int kk = (threadIdx.x >> 4) & 3;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int fc = __builtin_amdgcn_readlane(tl.fc, 16 * t);
+      const int base = __builtin_amdgcn_readlane(tl.le, 16 * t) * ROWS * ST;
+      const int col = tl.column(t, nfq);
+      const bool in = int(__builtin_amdgcn_readlane(v0, 16 * t)) >= 0;
+      ext[t] = in ? base + (E::NP + fc * NFP) * ST : -1;
+#pragma unroll
+      for (int s = 0; s < NK; ++s) {
+        const int k = 4 * s + kk, kc = fc * NFP + (k < NFP ? k : NFP - 1);
+        const double x = finterp[kc * nfq + col];
+        w[s][t] = k < NFP ? x : 0.0;
+        own[s][t] = base + s_fm[kc];
+      }
+    }
+  }
+  template <int C0, int NC, bool EXT>
+  __device__ __forceinline__ void interp(const double* s_n, double* out) const {
+    const int kk = (threadIdx.x >> 4) & 3;
+    QuadAcc<NC> acc;
+    acc.zero();
+#pragma unroll
+    for (int s = 0; s < NK; ++s) {
+      const int k = 4 * s + kk < NFP ? 4 * s + kk : NFP - 1;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int row = EXT && ext[t] >= 0 ? ext[t] + k * ST : own[s][t];
+        acc.step(t, s_n + C0 + row, w[s][t]);
+      }
+    }
+    acc.points(out);
+  }
+};
+
+// }}}
+
+// The gradients [NS][DIM] from the columns, which hold all but the energy's.
+template <int DIM, int NG>
+__device__ __forceinline__ void quad_gradients(const double* g, double* out) {
+#pragma unroll
+  for (int k = 0; k < DIM; ++k) out[DIM + k] = 0.0;   // not read
+#pragma unroll
+  for (int k = 0; k < NG; ++k) out[k < DIM ? k : k + DIM] = g[k];
+}
+
 // Temperature at a point with interpolated state q and seed.
 template <int DIM>
 __device__ __forceinline__ double ideal_temperature(const double* q, const GasDev& g) {
@@ -175,26 +392,34 @@ __device__ __forceinline__ double quad_point_temperature(const double* q, double
     return ideal_temperature<DIM>(q, g);
 }
 
-// The waves' tasks: volume points 64 at a time, then face points; the first
-// wave rotates with the block, so that two workgroups on a CU do not both
-// give their surplus task to the same SIMD.
-struct QuadTask {
-  bool face;
-  int t;   // point index among the workgroup's volume / face points, or -1
-};
-__device__ __forceinline__ int quad_task_count(int nvol, int nface) {
-  return (nvol + 63) / 64 + (nface + 63) / 64;
-}
-__device__ __forceinline__ QuadTask quad_task(int task, int nvol, int nface) {
-  const int nv = (nvol + 63) / 64;
-  QuadTask k;
-  k.face = task >= nv;
-  k.t = (k.face ? task - nv : task) * 64 + int(threadIdx.x & 63);
-  if (k.t >= (k.face ? nface : nvol)) k.t = -1;
-  return k;
+// The waves' tasks: volume points 64 at a time (3-D: four tiles of 16 points
+// of one element each), then face points; the first wave rotates with the
+// block, so that two workgroups on a CU do not both give their surplus task to
+// the same SIMD.
+template <bool MM>
+__device__ __forceinline__ int quad_task_count(int groups, int n) {
+  return MM ? (groups * ((n + 15) / 16) + 3) / 4 : (groups * n + 63) / 64;
 }
 __device__ __forceinline__ int quad_first_task() {
-  return ((threadIdx.x >> 6) + (blockIdx.x >> 3)) & (kWaves - 1);
+  return (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + (blockIdx.x >> 3)) & (kWaves - 1);
+}
+// The lane's point of a task; 2-D: 64 consecutive points, at most one tile.
+template <int DIM, int P>
+__device__ __forceinline__ QuadTiles<DIM, P> quad_point(bool face, int task, int ne, int n) {
+  if constexpr (DIM == 3) {
+    return QuadTiles<DIM, P>(face, task, ne, n);
+  } else {
+    QuadTiles<DIM, P> tl;
+    const int nf = face ? Elem<DIM, P>::NF : 1;
+    const int t = task * 64 + int(threadIdx.x & 63);
+    const int r = t / n;
+    tl.valid = t < ne * nf * n;
+    tl.m = t - r * n;
+    tl.le = r / nf;
+    tl.fc = r - tl.le * nf;
+    tl.m0 = 0;
+    return tl;
+  }
 }
 
 template <int DIM, int P, int NSP, int MIX>
@@ -223,38 +448,48 @@ __attribute__((amdgpu_waves_per_eu(2))) void ns_grad_quad_kernel(KArgs a, QuadAr
   // 2: state and temperature at the volume points; at the face points the
   // gradient flux value (central inside, the exterior value on boundaries)
   // times the face Jacobian ratio
-  const int ntask = quad_task_count(ne * nq, ne * nfq_all);
+  const int nvt = quad_task_count<C::MM>(ne, nq);
+  const int ntask = nvt + quad_task_count<C::MM>(ne * NF, nfq);
   for (int task = quad_first_task(); task < ntask; task += kWaves) {
-    const QuadTask tk = quad_task(task, ne * nq, ne * nfq_all);
-    if (tk.t < 0) continue;
-    if (!tk.face) {
-      const int le = tk.t / nq;
-      const int m = tk.t - le * nq;
-      double u[NQC];
-      quad_interp<NQC, NP>(qa.interp + m, nq, s_n + le * C::ROWS * ST, node, u);
+    const bool face = task >= nvt;
+    const auto tl = quad_point<DIM, P>(face, face ? task - nvt : task, ne, face ? nfq : nq);
+    if (!C::MM && !tl.valid) continue;
+    const int le = tl.le, m = tl.m;
+    const double* rows = s_n + le * C::ROWS * ST;
+    if (!face) {
+      double u[C::NC4];
+      if constexpr (C::MM)
+        quad_mm_volume<DIM, P, 0, C::NC4, ST, C::ROWS>(qa.interp, nq, tl, s_n, u);
+      else
+        quad_interp<NQC, NP>(qa.interp + m, nq, rows, node, u);
       const double tq = quad_point_temperature<DIM, NSP, MIX>(u, MIX ? u[NQC - 1] : 0.0,
                                                               a.gas, qa.niter);
+      if (!tl.valid) continue;
 #pragma unroll
       for (int f = 0; f < NFLD; ++f) s_u[(f * epb + le) * gs + m] = u[f];
       s_u[(NFLD * epb + le) * gs + m] = tq;
     } else {
-      const int le = tk.t / nfq_all;
-      const int rem = tk.t - le * nfq_all;
-      const int fc = rem / nfq;
-      const int m = rem - fc * nfq;
+      const int fc = tl.fc, rem = fc * nfq + m;
       const int64_t e = e0 + le;
       const int32_t v0 = a.vmap_p[(e * NF + fc) * NFP];
       const double sc = a.fscale[e * NF + fc];
-      double um[NQC], up[NQC];
-      const double* w = qa.finterp + fc * NFP * nfq + m;
-      const double* rows = s_n + le * C::ROWS * ST;
-      auto own = [&](int j) { return s_fm[fc * NFP + j]; };
+      double um[C::NC4], up[C::NC4];
+      if constexpr (C::MM) {
+        const QuadFaceTiles<DIM, P, ST, C::ROWS> ft(qa.finterp, nfq, tl, s_fm, v0);
+        ft.template interp<0, C::NC4, false>(s_n, um);
+        ft.template interp<0, C::NC4, true>(s_n, up);
+      } else {
+        const double* w = qa.finterp + fc * NFP * nfq + m;
+        if (v0 >= 0) {
+          quad_interp<NQC, NFP>(w, nfq, rows, [&](int j) { return s_fm[fc * NFP + j]; }, um);
+          quad_interp<NQC, NFP>(w, nfq, rows + (NP + fc * NFP) * ST, node, up);
+        }
+      }
+      if (!tl.valid) continue;
       double tp;
       if (v0 >= 0) {
-        quad_interp<NQC, NFP>(w, nfq, rows, own, um);
         const double tm = quad_point_temperature<DIM, NSP, MIX>(
             um, MIX ? um[NQC - 1] : 0.0, a.gas, qa.niter);
-        quad_interp<NQC, NFP>(w, nfq, rows + (NP + fc * NFP) * ST, node, up);
         tp = quad_point_temperature<DIM, NSP, MIX>(up, MIX ? up[NQC - 1] : 0.0, a.gas,
                                                    qa.niter);
 #pragma unroll
@@ -348,6 +583,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void ns_div_quad_kernel(KArgs a, QuadArg
   using C = QuadNs<DIM, P, NSP, MIX, true>;
   constexpr int NP = E::NP, NFP = E::NFP, NF = E::NF, ST = C::ST;
   constexpr int NFLD = C::NFLD, NSD = C::NSD, NQC = C::NQC, G0 = C::G0;
+  constexpr int NC4 = C::NC4, NC1 = C::NC1;
   extern __shared__ __align__(16) double lds16[];
   const int nq = qa.nq, nfq = qa.nfq, epb = qa.epb, nfq_all = NF * qa.nfq;
   const int gs = qa.gs, fs = qa.fs;
@@ -366,27 +602,34 @@ __attribute__((amdgpu_waves_per_eu(2))) void ns_div_quad_kernel(KArgs a, QuadArg
   __syncthreads();
   // 2: F_I - F_V at the volume points, in reference directions, and
   // F_I* - F_V* at the face points
-  const int ntask = quad_task_count(ne * nq, ne * nfq_all);
+  const int nvt = quad_task_count<C::MM>(ne, nq);
+  const int ntask = nvt + quad_task_count<C::MM>(ne * NF, nfq);
   for (int task = quad_first_task(); task < ntask; task += kWaves) {
-    const QuadTask tk = quad_task(task, ne * nq, ne * nfq_all);
-    if (tk.t < 0) continue;
-    if (!tk.face) {
-      const int le = tk.t / nq;
-      const int m = tk.t - le * nq;
-      const double* rows = s_n + le * C::ROWS * ST;
+    const bool face = task >= nvt;
+    const auto tl = quad_point<DIM, P>(face, face ? task - nvt : task, ne, face ? nfq : nq);
+    if (!C::MM && !tl.valid) continue;
+    const int le = tl.le, m = tl.m;
+    const double* rows = s_n + le * C::ROWS * ST;
+    // a point's columns: state, Newton seed, gradients
+    double col[C::NC4];
+    if (!face) {
       const double* w = qa.interp + m;
       Node<DIM, NSP> s;
-      {
-        double u[NQC];
-        quad_interp<NQC, NP>(w, nq, rows, node, u);
-        double tq = 0.0;
-        if constexpr (MIX != 0) tq = point_temperature<DIM, NSP>(u, u[NQC - 1], qa.niter);
+      if constexpr (C::MM)
+        quad_mm_volume<DIM, P, 0, NC1, ST, C::ROWS>(qa.interp, nq, tl, s_n, col);
+      else
+        quad_interp<NQC, NP>(w, nq, rows, node, col);
+      double tq = 0.0;
+      if constexpr (MIX != 0) tq = point_temperature<DIM, NSP>(col, col[NQC - 1], qa.niter);
 #pragma unroll
-        for (int f = 0; f < NFLD; ++f) s.q[f] = u[f];
-        node_state<DIM, NSP, MIX>(s, a.gas, tq);
-      }
+      for (int f = 0; f < NFLD; ++f) s.q[f] = col[f];
+      node_state<DIM, NSP, MIX>(s, a.gas, tq);
+      if constexpr (!C::MM)
+        quad_interp<C::NG, NP>(w, nq, rows + G0, node, col + G0);
+      else if constexpr (NC4 > NC1)
+        quad_mm_volume<DIM, P, NC1, NC4 - NC1, ST, C::ROWS>(qa.interp, nq, tl, s_n, col + NC1);
       double gacc[NSD], F[NFLD][DIM];
-      quad_interp<NSD, NP>(w, nq, rows + G0, node, gacc);
+      quad_gradients<DIM, C::NG>(col + G0, gacc);
       viscous_flux<DIM, NSP, MIX>(s, reinterpret_cast<const double(*)[DIM]>(gacc),
                                   gacc + NFLD * DIM, F);
       if (a.inviscid_on) {
@@ -402,6 +645,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void ns_div_quad_kernel(KArgs a, QuadArg
 #pragma unroll
           for (int d = 0; d < DIM; ++d) F[f][d] = -F[f][d];
       }
+      if (!tl.valid) continue;
       const double* rx = a.rx + (e0 + le) * DIM * DIM;
 #pragma unroll
       for (int f = 0; f < NFLD; ++f)
@@ -413,43 +657,51 @@ __attribute__((amdgpu_waves_per_eu(2))) void ns_div_quad_kernel(KArgs a, QuadArg
           s_g[(f * epb + le) * gs + r * nq + m] = g;
         }
     } else {
-      const int le = tk.t / nfq_all;
-      const int rem = tk.t - le * nfq_all;
-      const int fc = rem / nfq;
-      const int m = rem - fc * nfq;
+      const int fc = tl.fc, rem = fc * nfq + m;
       const int64_t e = e0 + le;
       const int32_t v0 = a.vmap_p[(e * NF + fc) * NFP];
-      const double* rows = s_n + le * C::ROWS * ST;
       double n[DIM];
 #pragma unroll
       for (int d = 0; d < DIM; ++d) n[d] = a.normals[(e * NF + fc) * DIM + d];
       const double* w = qa.finterp + fc * NFP * nfq + m;
       const int ext0 = (NP + fc * NFP) * ST;
       auto own = [&](int j) { return s_fm[fc * NFP + j]; };
+      using Tiles = QuadFaceTiles<DIM, P, ST, C::ROWS>;
+      std::conditional_t<C::MM, Tiles, int> ft;
+      if constexpr (C::MM) ft = Tiles(qa.finterp, nfq, tl, s_fm, v0);
       Node<DIM, NSP> sm, sp;
-      double fstar[NFLD], fv[NFLD];
+      double fstar[NFLD], fv[NFLD], gacc[NSD];
       // the own side's state and viscous flux first, then the other side's, so
       // that one gradient set is live
       {
-        double u[NQC], tm = 0.0, gacc[NSD];
-        quad_interp<NQC, NFP>(w, nfq, rows, own, u);
-        if constexpr (MIX != 0) tm = point_temperature<DIM, NSP>(u, u[NQC - 1], qa.niter);
+        double tm = 0.0;
+        if constexpr (C::MM)
+          ft.template interp<0, NC1, false>(s_n, col);
+        else
+          quad_interp<NQC, NFP>(w, nfq, rows, own, col);
+        if constexpr (MIX != 0) tm = point_temperature<DIM, NSP>(col, col[NQC - 1], qa.niter);
 #pragma unroll
-        for (int f = 0; f < NFLD; ++f) sm.q[f] = u[f];
+        for (int f = 0; f < NFLD; ++f) sm.q[f] = col[f];
         node_state<DIM, NSP, MIX>(sm, a.gas, tm);
-        quad_interp<NSD, NFP>(w, nfq, rows + G0, own, gacc);
+        if constexpr (!C::MM)
+          quad_interp<C::NG, NFP>(w, nfq, rows + G0, own, col + G0);
+        else if constexpr (NC4 > NC1)
+          ft.template interp<NC1, NC4 - NC1, false>(s_n, col + NC1);
+        quad_gradients<DIM, C::NG>(col + G0, gacc);
         viscous_flux_n<DIM, NSP, MIX>(sm, reinterpret_cast<const double(*)[DIM]>(gacc),
                                       gacc + NFLD * DIM, n, fv);
 #pragma unroll
         for (int f = 0; f < NFLD; ++f) fstar[f] = -0.5 * fv[f];
       }
+      // (boundary faces: the other side's gradient trace is the own one)
       double tp = 0.0;
+      if constexpr (C::MM)
+        ft.template interp<0, NC1, true>(s_n, col);
       if (v0 >= 0) {
-        double u[NQC];
-        quad_interp<NQC, NFP>(w, nfq, rows + ext0, node, u);
-        if constexpr (MIX != 0) tp = point_temperature<DIM, NSP>(u, u[NQC - 1], qa.niter);
+        if constexpr (!C::MM) quad_interp<NQC, NFP>(w, nfq, rows + ext0, node, col);
+        if constexpr (MIX != 0) tp = point_temperature<DIM, NSP>(col, col[NQC - 1], qa.niter);
 #pragma unroll
-        for (int f = 0; f < NFLD; ++f) sp.q[f] = u[f];
+        for (int f = 0; f < NFLD; ++f) sp.q[f] = col[f];
       } else {
         const int64_t bq = (-int64_t(v0) - 1) / NFP * nfq + m;
 #pragma unroll
@@ -462,17 +714,18 @@ __attribute__((amdgpu_waves_per_eu(2))) void ns_div_quad_kernel(KArgs a, QuadArg
 #pragma unroll
         for (int f = 0; f < NFLD; ++f) fstar[f] += fv[f];
       }
-      {
-        // the other side's gradient trace: the neighbour's (interior faces)
-        // or this element's own (boundary faces)
-        double gacc[NSD];
-        quad_interp<NSD, NFP>(
-            w, nfq, rows + G0, [&](int j) { return v0 >= 0 ? ext0 + j * ST : own(j); }, gacc);
-        viscous_flux_n<DIM, NSP, MIX>(sp, reinterpret_cast<const double(*)[DIM]>(gacc),
-                                      gacc + NFLD * DIM, n, fv);
+      if constexpr (!C::MM)
+        quad_interp<C::NG, NFP>(
+            w, nfq, rows + G0, [&](int j) { return v0 >= 0 ? ext0 + j * ST : own(j); },
+            col + G0);
+      else if constexpr (NC4 > NC1)
+        ft.template interp<NC1, NC4 - NC1, true>(s_n, col + NC1);
+      quad_gradients<DIM, C::NG>(col + G0, gacc);
+      viscous_flux_n<DIM, NSP, MIX>(sp, reinterpret_cast<const double(*)[DIM]>(gacc),
+                                    gacc + NFLD * DIM, n, fv);
 #pragma unroll
-        for (int f = 0; f < NFLD; ++f) fstar[f] -= 0.5 * fv[f];
-      }
+      for (int f = 0; f < NFLD; ++f) fstar[f] -= 0.5 * fv[f];
+      if (!tl.valid) continue;
       const double sc = a.fscale[e * NF + fc];
 #pragma unroll
       for (int f = 0; f < NFLD; ++f) s_f[(f * epb + le) * fs + rem] = -sc * fstar[f];
