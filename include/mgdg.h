@@ -345,9 +345,9 @@ mg_status mg_ns_rhs_quad(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* 
  *   ext_col[h][m]  = E[m][h]                       [nq][nfaces*nfq]
  *   apply_t[h][i]  = (M^-1 V_h^T)[i][h]            [nh][np]
  *   face_weights   = the face rule's weights       [nfq]
- * and the same operators along the cyclic diagonals (optional, used when
- * nq = 64 and nfaces*nfq = 192, i.e. 3-D p = 3 at degree 6, where each
- * two-point flux is then evaluated once for both of its rows):
+ * and the same operators along the cyclic diagonals (optional, used in 3-D
+ * when nq = (p + 1)^3 and nfq = 3 (p + 1)^2, the default rule of degree 2 p,
+ * where each two-point flux is then evaluated once for both of its rows):
  *   skew_diag[r][s][h] = (Q_r - Q_r^T)[h][(h + s) mod nq]   [dim][nq][nq]
  *   ext_diag[s][m]     = E[m][(m + s) mod nq]               [nq][nfaces*nfq] */
 typedef struct mg_esdg {
