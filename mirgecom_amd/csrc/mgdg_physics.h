@@ -164,70 +164,62 @@ __device__ __forceinline__ void mix_e_cv(double t, const double* y, double& e,
   cv = c_mech.gas_constant * sc;
 }
 
-// Internal energy of mass fractions y as a polynomial in T for one NASA7
-// range: e(T) = c[5] + T (c[0] + c[1] T + ... + c[4] T^4), and the gas
-// constant r; c_v(T) = c[0] + 2 c[1] T + ... + 5 c[4] T^4.
-template <int RANGE>
-__device__ __forceinline__ void mix_e_poly(const double* y, double* c, double& r) {
+// Internal energy of mass fractions y as a polynomial in T, every species in
+// the NASA7 range t lies in: e(T) = c[5] + T (c[0] + c[1] T + ... + c[4] T^4),
+// so that c_v(T) = c[0] + 2 c[1] T + ... + 5 c[4] T^4; r the gas constant of y.
+// A range that no lane of the wave needs is passed over, and a lane adds exact
+// zeros for the species of the other range: what it gets is the same in every
+// wave.
+__device__ __forceinline__ void mix_e_poly(double t, const double* y, double r, double* c) {
   PolyConst* poly = poly_here();
-  double s = 0.0;
+  double tmid_lo, tmid_hi;
+  nasa7_tmid_range(tmid_lo, tmid_hi);
 #pragma unroll
   for (int i = 0; i < 6; ++i) c[i] = 0.0;
+#pragma unroll 1
+  for (int range = 0; range < 2; ++range) {
+    if (!__any(range ? t > tmid_lo : !(t > tmid_hi))) continue;
 #pragma unroll
-  for (int k = 0; k < MIX_NSP; ++k) {
-    const double w = c_mech.inv_wt[k] * y[k];
-    const auto* h = poly->h[RANGE][k];
-    s += w;
+    for (int k = 0; k < MIX_NSP; ++k) {
+      const double w = (t > c_mech.t_mid[k]) == (range != 0) ? c_mech.inv_wt[k] * y[k] : 0.0;
+      const auto* h = poly->h[range][k];
 #pragma unroll
-    for (int i = 0; i < 6; ++i) c[i] += w * h[i];
+      for (int i = 0; i < 6; ++i) c[i] += w * h[i];
+    }
   }
 #pragma unroll
   for (int i = 0; i < 6; ++i) c[i] *= c_mech.gas_constant;
-  r = c_mech.gas_constant * s;
   c[0] -= r;
 }
 
 // Fixed-iteration Newton solve for T from mass-specific internal energy
-// (thermochemistry.py:126-167, update at :99-102).  When the whole wave is on
-// one side of every species' T_mid (the common case) the species are summed
-// into that range's polynomials once instead of in every update; a wave whose
-// lanes lie in both ranges updates by mix_e_cv.  Also c_v's coefficients cvp
-// of the range the result lies in (T_mid itself: the low one) and the gas
-// constant.  1.97 M nodes, 5 updates, on an MI355X: 132 -> 53 us (220 MB, 43 us
-// at the rate of a copy).
+// (thermochemistry.py:126-167, update at :99-102), with the species summed
+// into one polynomial before the updates and again only when a lane's T
+// changes its NASA7 range (or lies between the species' T_mid, where they
+// differ).  Also c_v's coefficients cvp of the range the result lies in (T_mid
+// itself: the low one) and the gas constant.  A node's result does not depend
+// on the nodes that share its wave.  MI355X, 5 updates, 1.97 M nodes (220 MB),
+// calls back to back: 38 us with all nodes in one range and 39 us across the
+// switch; with both ranges of every species in every update 118 and 167 us.
 __device__ __forceinline__ double mix_temperature_poly(double e_in, double t_seed,
                                                        const double* y, int niter,
                                                        double* cvp, double& r) {
   double tmid_lo, tmid_hi;
   nasa7_tmid_range(tmid_lo, tmid_hi);
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < MIX_NSP; ++k) s += c_mech.inv_wt[k] * y[k];
+  r = c_mech.gas_constant * s;
   double t = t_seed, c[6], d[5];
   int have = -1;
   for (int it = 0; it <= niter; ++it) {
-    const int want = __all(t > tmid_hi) ? 1 : (__all(!(t > tmid_lo)) ? 0 : 2);
-    if (want != have && want != 2) {
-      if (want == 1)
-        mix_e_poly<1>(y, c, r);
-      else
-        mix_e_poly<0>(y, c, r);
+    // 0 low, 1 high, 2 between
+    const int want = t > tmid_hi ? 1 : (t > tmid_lo ? 2 : 0);
+    if (__any(want != have || want == 2)) mix_e_poly(t, y, r, c);
+    have = want;
 #pragma unroll
-      for (int i = 0; i < 5; ++i) d[i] = (i + 1) * c[i];
-      have = want;
-    }
-    if (want == 2) {
-      // both ranges; the result's own afterwards
-      have = 2;
-      if (it == niter) {
-        double ch[6];
-        mix_e_poly<1>(y, ch, r);
-        mix_e_poly<0>(y, c, r);
-#pragma unroll
-        for (int i = 0; i < 5; ++i) d[i] = (i + 1) * (t > tmid_hi ? ch[i] : c[i]);
-      } else {
-        double e, cv;
-        mix_e_cv(t, y, e, cv);
-        t = t + (e_in - e) / cv;
-      }
-    } else if (it < niter) {
+    for (int i = 0; i < 5; ++i) d[i] = (i + 1) * c[i];
+    if (it < niter) {
       const double e = c[5] + t * (c[0] + t * (c[1] + t * (c[2] + t * (c[3] + t * c[4]))));
       t = t + (e_in - e) / horner5(d, t);
     }
@@ -246,7 +238,8 @@ __device__ __forceinline__ double mix_temperature(double e_in, double t_seed,
 // Newton solve to a tolerance: iterate T <- T + (e - e(T))/cv(T) until the
 // update is at most tol (checked after each update) or max_iter updates;
 // *iters receives the number of updates, or -1 when the last update still
-// exceeded tol.  The update is the fixed-iteration solve's (mix_e_cv).
+// exceeded tol.  e(T) and c_v(T) are summed species by species (mix_e_cv) in
+// every update; the fixed-iteration solve's polynomial rounds differently.
 __device__ __forceinline__ double mix_temperature_tol(double e_in, double t_seed,
                                                       const double* y, double tol,
                                                       int max_iter, int* iters) {
