@@ -51,6 +51,7 @@ struct EsdgPairs {
   static constexpr int G = NFT / NQ;
   static constexpr int GPW = 64 / NQ;
   static constexpr int EPB = GPW;            // elements per workgroup
+  static constexpr int SPAN = GPW > 4 ? 256 / GPW : 64;   // a wave's lanes to an element
   static constexpr int NB = P == 3 ? 1 : (P == 2 && MIX) ? 4 : 2;
   static constexpr int RT = G / NB;
   static constexpr int NC = 4 / NB;
@@ -138,7 +139,7 @@ __device__ __forceinline__ void esdg_pair_rows(const KArgs& a, const EsdgArgs& e
       LnPair ln[RT];
 #pragma unroll
       for (int r = 0; r < RT; ++r) flux.begin(pm[r], pj, ln[r]);
-      ln_means<Flux::SHORT>(ln, [&](int r, double& e1, double& e2) {
+      ln_means<Flux::SHORT, C::SPAN>(ln, [&](int r, double& e1, double& e2) {
         const double* lm = lg + Flux::LOGS * (NQ + (blk + r) * NQ + l);
         const double* lj = lg + Flux::LOGS * j;
         e1 = lj[0] - lm[0];
@@ -223,7 +224,7 @@ __device__ __forceinline__ void esdg_pair_rows(const KArgs& a, const EsdgArgs& e
       double rho, eng, prm, un = 0.0;
       LnPair ln[1];
       flux.begin(ph, pj, ln[0]);
-      ln_means<Flux::SHORT>(ln, [&](int, double& e1, double& e2) {
+      ln_means<Flux::SHORT, C::SPAN>(ln, [&](int, double& e1, double& e2) {
         e1 = lg[Flux::LOGS * j] - lg[Flux::LOGS * l];
         e2 = lg[Flux::LOGS * j + Flux::LOG2] - lg[Flux::LOGS * l + Flux::LOG2];
       });
@@ -511,7 +512,8 @@ __device__ __forceinline__ void ec_face_flux(const EcPrim<3, NSP>& m, const EcPr
   const EcPaired<3, NSP> flux(gamma);
   LnPair ln[1];
   flux.begin(m, p, ln[0]);
-  ln_means<true>(ln, [&](int, double& e1, double& e2) {
+  // (the long series: the wave's other points belong to other elements)
+  ln_means<false, 64>(ln, [&](int, double& e1, double& e2) {
     e1 = p.lrho - m.lrho;
     e2 = p.lbeta - m.lbeta;
   });
@@ -841,7 +843,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void esdg_mix_pair_kernel(KArgs a, EsdgA
           const RnPaired<3, false> flux;
           LnPair ln[1];
           flux.begin(own.pt, s.pt, ln[0]);
-          ln_means<false>(ln, [&](int, double& e1, double& e2) {
+          ln_means<false, 64>(ln, [&](int, double& e1, double& e2) {
             e1 = s.pt.lrho[0] - own.pt.lrho[0];
             e2 = s.pt.lth - own.pt.lth;
           });

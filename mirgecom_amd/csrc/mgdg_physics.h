@@ -752,12 +752,12 @@ __device__ __forceinline__ void ec_flux_dot(const EcPairLog<DIM, NSP>& a,
 // With z = (x - y) / (x + y) and f = z^2, ln x - ln y = 2 artanh z, so that
 //   ln-mean(x, y)     = (x + y) / 2 * P(f),  P = z / artanh z
 //   1 / ln-mean(x, y) = 2 / (x + y) * Q(f),  Q = artanh z / z = sum f^k / (2k + 1)
-// N + 1 terms leave a relative error below f^(N+1): 3e-18 for N = 3 at
-// f < 1e-4 (the reference's threshold) and 3e-17 for N = 9 at f < 3e-2.  The
-// loop takes the short series when all of a wave's pairs allow it (SHORT; the
-// mixture's pairs seldom do, and go to the long one at once), the long one
-// otherwise, and the logarithms themselves only in waves with a pair beyond
-// 3e-2 (values 42 % apart).
+// N + 1 terms leave a relative error of f^(N+1) / (2 N + 3) in Q and less in
+// P: 1e-17 for N = 3 at f < 1e-4 (the reference's threshold) and
+// 3e-17 for N = 9 at f < 3e-2.  The loop takes the short series when all of an
+// element's pairs allow it that a wave holds (SHORT; the mixture's pairs seldom
+// do, and go to the long one at once), the long one otherwise, and the
+// logarithms themselves for pairs beyond 3e-2 (values 42 % apart).
 constexpr double kLnNear = 1e-4, kLnFar = 3e-2;
 constexpr int kLnShort = 3, kLnLong = 9;
 
@@ -804,15 +804,25 @@ struct LnPair {
   }
 };
 
+// Whether p holds on all of a lane's SPAN neighbours (32: its half of the
+// wave, all of whose lanes are active).
+template <int SPAN>
+__device__ __forceinline__ bool ln_all(bool p) {
+  static_assert(SPAN == 64 || SPAN == 32, "lanes");
+  if constexpr (SPAN == 64) return __all(p);
+  return unsigned(__ballot(p) >> (threadIdx.x & 32)) == ~0u;
+}
+
 // The means of R pairs at once (one branch, and the pairs' chains of
 // operations interleave); far(r, e1, e2) gives ln y - ln x of both
-// quantities of pair r.
-template <bool SHORT, int R, typename Far>
+// quantities of pair r.  SPAN: the lanes that work on one element, whose
+// series so does not depend on the element beside it in the wave.
+template <bool SHORT, int SPAN, int R, typename Far>
 __device__ __forceinline__ void ln_means(LnPair (&a)[R], Far far) {
   double fm = 0.0, p[R], q[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) fm = fmax(fm, fmax(a[r].f1, a[r].f2));
-  bool all = SHORT && __all(fm < kLnNear);
+  bool all = SHORT && ln_all<SPAN>(fm < kLnNear);
   if (all) {
 #pragma unroll
     for (int r = 0; r < R; ++r) ln_pq<kLnShort>(a[r].f1, a[r].f2, p[r], q[r]);
