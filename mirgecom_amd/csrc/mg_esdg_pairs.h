@@ -67,6 +67,15 @@ struct EsdgPairs {
     return reinterpret_cast<Pt*>(reinterpret_cast<D*>(s_pt) +
                                  le * (int(sizeof(Pt)) / 8 * NH + PAD));
   }
+  // lane group and element of a thread (lanes past GPW * NQ repeat the first
+  // group's first lane and store nothing)
+  static __device__ __forceinline__ int group() {
+    const int wl = threadIdx.x & 63;
+    return wl < GPW * NQ ? wl / NQ : 0;
+  }
+  static __device__ __forceinline__ int element() {
+    return ((threadIdx.x >> 6) * GPW + group()) >> 2;
+  }
   static_assert(G * NQ == NFT && RT * NB == G && kWaves == 4, "row groups");
 };
 
@@ -81,14 +90,12 @@ __device__ __forceinline__ void esdg_pair_rows(const KArgs& a, const EsdgArgs& e
   constexpr int DIM = 3, NF = DIM + 1, NFLD = Flux::NFLD, NSP = Flux::NSP, NV = 2 + DIM;
   constexpr int NQ = C::NQ, NFT = C::NFT, RT = C::RT, NC = C::NC;
   using Pt = typename Flux::Point;
-  const int wl = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // lanes past GPW * NQ repeat lane 0's work and store nothing
+  const int wl = threadIdx.x & 63;
   const bool lane_on = wl < C::GPW * NQ;
-  const int sub = lane_on ? wl / NQ : 0;
+  const int sub = C::group();
   const int l = lane_on ? wl - sub * NQ : 0;
   const int base = sub * NQ;
-  const int slot = wave * C::GPW + sub;
-  const int le = slot >> 2, sq = slot & 3;
+  const int le = C::element(), sq = ((threadIdx.x >> 6) * C::GPW + sub) & 3;
   const int64_t e = le < ne ? e0 + le : e0;
   const Pt* pt = C::points(s_pt, le);
   const double* lg = Flux::LOGS == 2 ? s_log + le * C::NH * 2
@@ -840,7 +847,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void esdg_mix_pair_kernel(KArgs a, EsdgA
           own = s;
         } else {
           double rho, eng, prm, un = 0.0;
-          const RnPaired<3, false> flux;
+          const RnPaired<3, false> flux(false);
           LnPair ln[1];
           flux.begin(own.pt, s.pt, ln[0]);
           ln_means<false, 64>(ln, [&](int, double& e1, double& e2) {
@@ -874,17 +881,20 @@ __attribute__((amdgpu_waves_per_eu(2))) void esdg_mix_pair_kernel(KArgs a, EsdgA
     }
   }
   __syncthreads();
-  // 3: rows of (Q_h - Q_h^T) o F_S, plus the face flux on face rows: the
-  // points' c_v polynomials where every element of the workgroup keeps to one
-  // NASA7 range
+  // 3: rows of (Q_h - Q_h^T) o F_S, plus the face flux on face rows: the loop
+  // without the sums over species where every element of the workgroup keeps
+  // to one NASA7 range
   bool poly = true;
   for (int le = 0; le < ne; ++le) poly = poly && s_rng[le] != 0;
+  const bool own_poly = s_rng[C::element()] != 0;
   constexpr int LOG0 = offsetof(Pt, lrho) / sizeof(double);
   static_assert(sizeof(Pt) == 22 * 8 && offsetof(Pt, lth) == 8 * (LOG0 + 8), "point layout");
   if (poly)
-    esdg_pair_rows<P, true>(a, ea, RnPaired<3, true>(), s_pt, nullptr, LOG0, s_fs, lds16, e0, ne);
+    esdg_pair_rows<P, true>(a, ea, RnPaired<3, true>(true), s_pt, nullptr, LOG0, s_fs, lds16, e0,
+                            ne);
   else
-    esdg_pair_rows<P, true>(a, ea, RnPaired<3, false>(), s_pt, nullptr, LOG0, s_fs, lds16, e0, ne);
+    esdg_pair_rows<P, true>(a, ea, RnPaired<3, false>(own_poly), s_pt, nullptr, LOG0, s_fs, lds16,
+                            e0, ne);
   // 4: dQ/dt = -M^-1 V_h^T acc
   esdg_pair_apply<P, true, NFLD>(a, ea, lds16, s_n, e0, ne);
 }

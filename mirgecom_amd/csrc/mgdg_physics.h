@@ -1018,9 +1018,11 @@ __device__ __forceinline__ void rn_flux_dot(const RnPair<DIM>& a, const RnPair<D
 }
 
 // rn_flux_dot for the paired loop (see EcPaired; e = c_v(T_mean) T_mean +
-// u_a . u_b / 2).  POLY: every point of the element lies in one NASA7 range,
-// and so does T_mean, which lies between the two temperatures: c_v comes from
-// the points' polynomials.
+// u_a . u_b / 2).  Where both points lie in one NASA7 range (one), so does
+// T_mean, which lies between their temperatures, and c_v comes from the points'
+// polynomials; a lane with points of both ranges sums the species.  POLY: no
+// lane's points do.  Either form gives a lane with points of one range the same
+// result.
 template <int DIM, bool POLY>
 struct RnPaired {
   static constexpr int NSP = MIX_NSP;
@@ -1029,6 +1031,8 @@ struct RnPaired {
   static constexpr bool SHORT = false;
   static constexpr int NFLD = 2 + DIM + NSP;
   using Point = RnPoint<DIM>;
+  bool one;
+  __device__ __forceinline__ explicit RnPaired(bool one_range) : one(one_range) {}
   __device__ __forceinline__ static void begin(const Point& a, const Point& b, LnPair& l) {
     l.s1 = a.rhoh + b.rhoh;
     l.d1 = a.rhoh - b.rhoh;
@@ -1044,17 +1048,17 @@ struct RnPaired {
     double uu = 0.0;
 #pragma unroll
     for (int d = 0; d < DIM; ++d) uu += a.uh[d] * b.uh[d];
-    double cvm;
-    if constexpr (POLY) {
-      double c[5];
+    double c[5];
 #pragma unroll
-      for (int i = 0; i < 5; ++i) c[i] = a.cv[i] + b.cv[i];
-      cvm = horner5(c, t_mean);
-    } else {
-      double y[MIX_NSP];
+    for (int i = 0; i < 5; ++i) c[i] = a.cv[i] + b.cv[i];
+    double cvm = horner5(c, t_mean);
+    if constexpr (!POLY) {
+      if (!one) {
+        double y[MIX_NSP];
 #pragma unroll
-      for (int k = 0; k < MIX_NSP; ++k) y[k] = a.yh[k] + b.yh[k];
-      cvm = mix_cv(t_mean, y);
+        for (int k = 0; k < MIX_NSP; ++k) y[k] = a.yh[k] + b.yh[k];
+        cvm = mix_cv(t_mean, y);
+      }
     }
     e = fma(2.0, uu, cvm * t_mean);
   }

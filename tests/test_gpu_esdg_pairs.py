@@ -3,8 +3,9 @@ flux once, for both rows) against the row-by-row kernels, which run when
 ``mg_esdg`` carries no diagonal layouts: p = 1..3 on element counts that leave
 the last workgroup ragged, both gases, smooth and far states -- densities up
 to a factor of four apart inside an element (the logarithmic means' long
-series and logarithms) and temperatures across the NASA7 switch (elements
-without one range for all points) -- and prescribed boundaries.
+series and logarithms), projected temperatures across the NASA7 switch
+(elements without one range for all points, beside others with one) -- and
+dummy boundaries.
 
 Both orders of summation agree to the states' own rounding: fluxes p/rho ~ 1
 (ideal) or ~1e5 J/m^3 (mixture) enter a difference of ~1e2 terms with
@@ -17,6 +18,7 @@ import pytest
 torch = pytest.importorskip("torch")
 
 from tests.cases import Problem, mixture_state, rel_err, smooth_perturbed_state  # noqa: E402
+from tests.test_gpu_element_order import bump_state  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -54,12 +56,22 @@ def _both(pb, q, t, bnd):
 @pytest.mark.parametrize("order", [1, 2, 3])
 @pytest.mark.parametrize("gas,far", [("ideal", False), ("ideal", True),
                                      ("species", True), ("mixture", False),
-                                     ("mixture", True)])
+                                     ("mixture", True), ("switch", True)])
 def test_paired_matches_rows(order, gas, far):
     print(f"paired esdg p={order} {gas} far={far}", flush=True)
-    pb = Problem(3, order, (3, 5, 3), 0.0, (2.0, 2.1, 1.9), (True,) * 3)
+    box = 1.0 if gas == "switch" else (2.0, 2.1, 1.9)
+    pb = Problem(3, order, (3, 5, 3), 0.0, box, (True,) * 3)
     t = None
-    if gas == "mixture":
+    if gas == "switch":
+        # the entropy-stable projection's temperatures lie several hundred
+        # kelvin above the state's (no formation energy in p / (gamma - 1))
+        from oracle import esdg, physics as ph, thermochem as tc
+        q, t = bump_state(pb.x, "mixture")
+        tp = esdg._es_projected_state(q, t, ph.GasModel(tc.PyrometheusMixture(5)),
+                                      3).temperature
+        cross = (tp.min(1) < 950.0) & (tp.max(1) > 1050.0)
+        assert cross.any() and (tp.min(1) > 1050.0).any()
+    elif gas == "mixture":
         q, t = mixture_state(pb.x, 5, t_mean=1100.0 if far else 1700.0,
                              t_amp=600.0 if far else 200.0)
     else:
