@@ -84,11 +84,12 @@ def _nasa7(t, coef_lo, coef_hi):
 
 
 def source_buffer(q, dim):
-    """A buffer like ``q`` for species sources, zero outside the species rows,
-    every one of which the source kernels write.  From 2**17 nodes on only the
-    zero rows are filled, 15 us less at 1.97 M nodes; below, where the host's
-    calls count, one fill of everything saves two of them, 1 us of 78."""
-    if q.numel() < q.shape[0] << 17:
+    """A buffer like ``q`` for species sources, zero outside the mechanism's
+    species rows, every one of which the source kernels write.  From 2**17 nodes
+    on only the zero rows are filled, 15 us less at 1.97 M nodes; below, where
+    the host's calls count, one fill of everything saves two of them, 1 us of
+    78.  A state with further rows is filled whole too."""
+    if q.numel() < q.shape[0] << 17 or q.shape[0] != 2 + dim + mech.NSPECIES:
         return torch.zeros_like(q)
     out = torch.empty_like(q)
     out[:2 + dim].zero_()

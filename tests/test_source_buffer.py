@@ -1,16 +1,59 @@
-"""``eos.source_buffer``: the rows outside the species are zero on both sides of
-the size from which only they are filled, and the buffer is the state's."""
+"""``eos.source_buffer``: the rows that the source kernels do not write are zero
+on both sides of the size from which only they are filled, whatever memory the
+buffer is made of, also for a state with more rows than the mechanism's; and
+the kernels write all others."""
 
 import pytest
 
 torch = pytest.importorskip("torch")
 
 
+def _poison(monkeypatch):
+    monkeypatch.setattr(torch, "empty_like",
+                        lambda q, **kw: torch.full_like(q, float("nan"), **kw))
+
+
+@pytest.mark.parametrize("extra", [0, 2])
 @pytest.mark.parametrize("dim", [2, 3])
 @pytest.mark.parametrize("nodes", [0, 1, (1 << 17) - 1, 1 << 17])
-def test_zero_rows(dim, nodes):
+def test_zero_rows(monkeypatch, nodes, dim, extra):
     from mirgecom_amd.eos import source_buffer
-    q = torch.ones((9 + dim, nodes, 1), dtype=torch.float64)
+    _poison(monkeypatch)
+    q = torch.ones((9 + dim + extra, nodes, 1), dtype=torch.float64)
     out = source_buffer(q, dim)
     assert out.shape == q.shape and out.dtype == q.dtype and out.is_contiguous()
-    assert not out[:2 + dim].any() and out.data_ptr() != q.data_ptr() or nodes == 0
+    assert nodes == 0 or out.data_ptr() != q.data_ptr()
+    assert (out[:2 + dim] == 0).all()
+    assert (out[9 + dim:] == 0).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("extra", [0, 2])
+@pytest.mark.parametrize("nel", [13107, 13110])   # 131,070 and 131,100 nodes
+def test_kernels_write_every_species_row(monkeypatch, nel, extra):
+    from mirgecom_amd.eos import PyrometheusMixture
+    from mirgecom_amd.fluid import ConservedVars
+    from mirgecom_amd.surrogate import ChemistrySurrogate
+    print(f"source buffer nel={nel} extra={extra}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(nel)
+    y = 0.05 + torch.rand((7, nel, 10), generator=gen, dtype=torch.float64,
+                          device="cuda")
+    rho = 0.1 + 0.05 * torch.rand((nel, 10), generator=gen, dtype=torch.float64,
+                                  device="cuda")
+    q = torch.zeros((12 + extra, nel, 10), dtype=torch.float64, device="cuda")
+    q[0], q[5:12] = rho, rho * y / y.sum(0)
+    temp = 1500.0 + 500.0 * y[0]
+    model = ChemistrySurrogate(device="cuda")
+    nm = model.norm
+    for i in range(10):
+        nm.in_mean[i], nm.in_scale[i] = 0.0, 1.0
+        nm.lo[i], nm.hi[i] = -1e300, 1e300
+    for i in range(7):
+        nm.out_mean[i], nm.out_scale[i] = 0.0, 1e-6
+    nm.sample_period = 0
+    cv = ConservedVars(3, q)
+    _poison(monkeypatch)
+    for src in (PyrometheusMixture().get_species_source_terms(cv, temp).q,
+                model.species_source(cv, temp, 1e-8, 10).q):
+        assert torch.isfinite(src[5:12]).all()
+        assert (src[:5] == 0).all() and (src[12:] == 0).all()
