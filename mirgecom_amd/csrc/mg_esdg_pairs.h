@@ -502,7 +502,6 @@ __device__ __forceinline__ void ec_state(const double* ref, const double* d, dou
   s.beta = 0.5 * w;
   s.kh = 0.25 * u2;
   s.rho = ref[0] * exp(x);
-  s.rhoh = 0.5 * s.rho;
   s.p = s.rho * iw;
   s.c = sqrt(u2) + sqrt(gamma * iw);
   if constexpr (NSP > 0)
@@ -517,14 +516,15 @@ __device__ __forceinline__ void ec_face_flux(const EcPrim<3, NSP>& m, const EcPr
                                              double sc, double* out) {
   double rho, eng, prm, un = 0.0;
   const EcPaired<3, NSP> flux(gamma);
+  const EcPair<3, NSP> pm(m), pp(p);
   LnPair ln[1];
-  flux.begin(m, p, ln[0]);
+  flux.begin(pm, pp, ln[0]);
   // (the long series: the wave's other points belong to other elements)
   ln_means<false, 64>(ln, [&](int, double& e1, double& e2) {
     e1 = p.lrho - m.lrho;
     e2 = p.lbeta - m.lbeta;
   });
-  flux.finish(m, p, ln[0], rho, eng, prm);
+  flux.finish(pm, pp, ln[0], rho, eng, prm);
 #pragma unroll
   for (int i = 0; i < 3; ++i) un += n[i] * (m.uh[i] + p.uh[i]);
   const double mass = rho * un;

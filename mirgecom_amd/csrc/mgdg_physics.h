@@ -629,29 +629,29 @@ __device__ __forceinline__ void entropy_to_cons(const double* ev, double gamma,
   for (int k = 0; k < NSP; ++k) q[2 + DIM + k] = mass * (ev[2 + DIM + k] * gm1);
 }
 
+// Per-point quantities of the entropy-conserving flux, with the logarithms
+// of rho and beta = rho/(2p) taken once per point.
 template <int NSP>
 struct EcSpecies {
   double yh[NSP];  // Y / 2
 };
+// Without species one padding double makes a 3-D point 9 doubles: an odd
+// stride in 8-byte words, so that lanes reading consecutive points from LDS
+// spread over the banks (8 doubles put 64 lanes on 4 bank groups).  With species
+// a 2-D point is 14 doubles; 16 put every fourth lane on the same banks (2-D
+// p = 2, 4,608 triangles: 59 us instead of 45).
 template <>
-struct EcSpecies<0> {};
-
-// What the paired two-point flux reads of a point (kept in LDS per hybridized
-// point).  16-byte aligned for 16-byte LDS reads; in 3-D a point is 6 (14
-// with species) doubles, so that the 16 lanes of one read phase fall into
-// different banks.
-template <int DIM, int NSP>
-struct alignas(16) EcPair : EcSpecies<NSP> {
-  double rhoh;     // rho / 2
-  double beta;
-  double uh[DIM];  // u / 2
+struct EcSpecies<0> {
+  double pad_;
 };
 
-// ... with rho, |u|^2 / 4 and the logarithms of rho and beta.
+// What the two-point flux of the row-by-row kernels reads of a point (kept in
+// LDS per hybridized point).
 template <int DIM, int NSP>
-struct EcPairLog : EcPair<DIM, NSP> {
-  double rho, kh;
-  double lrho, lbeta;
+struct EcPairLog : EcSpecies<NSP> {
+  double rho, lrho, beta, lbeta;
+  double kh;       // |u|^2 / 4
+  double uh[DIM];  // u / 2
 };
 
 // ... with the pressure and the wavespeed |u| + c the face flux needs.
@@ -660,11 +660,36 @@ struct EcPrim : EcPairLog<DIM, NSP> {
   double p, c;
 };
 
+// What the paired two-point flux reads of a point (kept in LDS per hybridized
+// point).  16-byte aligned for 16-byte LDS reads; in 3-D a point is 6 doubles
+// (an odd number of 16-byte words: the 16 lanes of one read phase fall into
+// different banks), with species 12.
+template <int NSP>
+struct EcPairSpecies {
+  double yh[NSP];
+};
+template <>
+struct EcPairSpecies<0> {};
+template <int DIM, int NSP>
+struct alignas(16) EcPair : EcPairSpecies<NSP> {
+  double rhoh;     // rho / 2
+  double beta;
+  double uh[DIM];  // u / 2
+  EcPair() = default;
+  __device__ __forceinline__ EcPair(const EcPrim<DIM, NSP>& s) : rhoh(0.5 * s.rho), beta(s.beta) {
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) uh[d] = s.uh[d];
+    if constexpr (NSP > 0) {
+#pragma unroll
+      for (int k = 0; k < NSP; ++k) this->yh[k] = s.yh[k];
+    }
+  }
+};
+
 template <int DIM, int NSP>
 __device__ __forceinline__ void ec_prim(const double* q, double gamma,
                                         EcPrim<DIM, NSP>& a) {
   a.rho = q[0];
-  a.rhoh = 0.5 * q[0];
   const double irho = 1.0 / q[0];
   double u2 = 0.0;
 #pragma unroll
@@ -946,8 +971,8 @@ struct RnPair {
 };
 
 // ... in the paired loop: with half of the point's part of the mixture c_v as
-// a polynomial in T (the NASA7 range the point lies in).  22 doubles in 3-D:
-// 4 mod 8 dwords, as EcPair.
+// a polynomial in T (the NASA7 range the point lies in).  22 doubles in 3-D,
+// an odd number of 16-byte words (see EcPair).
 template <int DIM>
 struct alignas(16) RnPoint {
   double rhoh, th;    // rho / 2, 1 / T
