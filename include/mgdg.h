@@ -347,7 +347,8 @@ mg_status mg_ns_rhs_quad(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* 
  *   face_weights   = the face rule's weights       [nfq]
  * and the same operators along the cyclic diagonals (optional, used in 3-D
  * when nq = (p + 1)^3 and nfq = 3 (p + 1)^2, the default rule of degree 2 p,
- * where each two-point flux is then evaluated once for both of its rows):
+ * and, without a mixture, when nq = 64 and nfq = 48; each two-point flux is
+ * then evaluated once for both of its rows):
  *   skew_diag[r][s][h] = (Q_r - Q_r^T)[h][(h + s) mod nq]   [dim][nq][nq]
  *   ext_diag[s][m]     = E[m][(m + s) mod nq]               [nq][nfaces*nfq] */
 typedef struct mg_esdg {

@@ -1,7 +1,8 @@
-// Entropy-stable (flux-differencing) Euler kernels of 3-D elements with the
-// default quadrature: nq = (p+1)^3 volume and 12 (p+1)^2 face points.  Each
-// two-point flux is evaluated once, for both of its rows; other rules and 2-D
-// take the row-by-row kernels (mgdg_kernels.h).
+// Entropy-stable (flux-differencing) Euler kernels of 3-D elements with a
+// quadrature of (Q+1)^3 volume and 12 (Q+1)^2 face points: the default one (Q = p)
+// and, without a mixture, Q = 3 at every order.  Each two-point flux is evaluated
+// once, for both of its rows; other rules and 2-D take the row-by-row kernels
+// (mgdg_kernels.h).
 //
 // Measured on an MI355X (kernel with the projection, before -> after this
 // layout): ideal gas p = 3, 82,944 tets 6.1 -> 4.4 ms; uiuc_7sp mixture
@@ -42,23 +43,23 @@ namespace mgdg {
 // took 7.5 ms.  The sums stay in registers until all of the
 // workgroup's pairs are done and then go over the points' LDS: four pieces
 // of the volume rows, NC of the face rows, added before the last phase.
-template <int P, bool MIX>
+template <int Q, bool MIX>
 struct EsdgPairs {
-  static constexpr int NQ = (P + 1) * (P + 1) * (P + 1);
-  static constexpr int NFQ = 3 * (P + 1) * (P + 1);
+  static constexpr int NQ = (Q + 1) * (Q + 1) * (Q + 1);
+  static constexpr int NFQ = 3 * (Q + 1) * (Q + 1);
   static constexpr int NFT = 4 * NFQ;
   static constexpr int NH = NQ + NFT;
   static constexpr int G = NFT / NQ;
   static constexpr int GPW = 64 / NQ;
   static constexpr int EPB = GPW;            // elements per workgroup
   static constexpr int SPAN = GPW > 4 ? 256 / GPW : 64;   // a wave's lanes to an element
-  static constexpr int NB = P == 3 ? 1 : (P == 2 && MIX) ? 4 : 2;
+  static constexpr int NB = Q == 3 ? 1 : (Q == 2 && MIX) ? 4 : 2;
   static constexpr int RT = G / NB;
   static constexpr int NC = 4 / NB;
   static constexpr int NACC = 4 * NQ + NC * NFT;   // row sums per field
   // doubles between two elements' points past the points themselves: at p = 2
   // a wave's two lane groups then read as one run of points (LDS banks)
-  static constexpr int PAD = P == 2 ? 24 : 0;
+  static constexpr int PAD = Q == 2 ? 24 : 0;
   template <class Pt>
   static constexpr int POINTS = EPB * (int(sizeof(Pt)) / 8 * NH + PAD);
   template <class Pt>
@@ -79,14 +80,14 @@ struct EsdgPairs {
   static_assert(G * NQ == NFT && RT * NB == G && kWaves == 4, "row groups");
 };
 
-template <int P, bool MIX, class Flux>
+template <int Q, bool MIX, class Flux>
 __device__ __forceinline__ void esdg_pair_rows(const KArgs& a, const EsdgArgs& ea,
                                                const Flux& flux,
                                                const typename Flux::Point* s_pt,
                                                const double* s_log, int s_off,
                                                const double* s_fs,
                                                double* s_acc, int64_t e0, int ne) {
-  using C = EsdgPairs<P, MIX>;
+  using C = EsdgPairs<Q, MIX>;
   constexpr int DIM = 3, NF = DIM + 1, NFLD = Flux::NFLD, NSP = Flux::NSP, NV = 2 + DIM;
   constexpr int NQ = C::NQ, NFT = C::NFT, RT = C::RT, NC = C::NC;
   using Pt = typename Flux::Point;
@@ -303,9 +304,9 @@ __device__ __forceinline__ void esdg_pair_rows(const KArgs& a, const EsdgArgs& e
 // and its reads are all in flight together (lanes over outputs, a quarter of
 // the rows per wave, waited on the operator eight reads at a time); s_part
 // holds the SPL partial results.
-template <int P, bool MIX, int NFLD>
+template <int P, int Q, bool MIX, int NFLD>
 struct EsdgApply {
-  using C = EsdgPairs<P, MIX>;
+  using C = EsdgPairs<Q, MIX>;
   static constexpr int NP = Elem<3, P>::NP;
   static constexpr int FS = NFLD > 6 ? 2 : 1;
   static constexpr int FL = (NFLD + FS - 1) / FS;
@@ -316,12 +317,12 @@ struct EsdgApply {
   static_assert(FL * FS == NFLD && SPL >= 1, "fields per lane");
 };
 
-template <int P, bool MIX, int NFLD>
+template <int P, int Q, bool MIX, int NFLD>
 __device__ __forceinline__ void esdg_pair_apply(const KArgs& a, const EsdgArgs& ea,
                                                 double* s_acc, double* s_part, int64_t e0,
                                                 int ne) {
-  using C = EsdgPairs<P, MIX>;
-  using A = EsdgApply<P, MIX, NFLD>;
+  using C = EsdgPairs<Q, MIX>;
+  using A = EsdgApply<P, Q, MIX, NFLD>;
   constexpr int NP = A::NP, NQ = C::NQ, NFT = C::NFT, NH = C::NH;
   constexpr int FS = A::FS, FL = A::FL, SPL = A::SPL, RPL = A::RPL;
   const int split = threadIdx.x / A::GRP;
@@ -397,28 +398,28 @@ __device__ __forceinline__ void esdg_pair_apply(const KArgs& a, const EsdgArgs& 
 // the first node so that nothing is lost to the size of the exponents.  The
 // interior states took 24,000 cycles per workgroup with the powers, 16,000 so.
 
-template <int P, int STRIDE>
+template <int P, int Q, int STRIDE>
 struct EsdgNodes {
   using E = Elem<3, P>;
-  using C = EsdgPairs<P, false>;
+  using C = EsdgPairs<Q, false>;
   static constexpr int ROWS = E::NP + E::NFN + 1;
   static constexpr int SIZE = C::EPB * ROWS * STRIDE;
 };
 
 // Element le's nodal values: rows 0..NP-1 own nodes, then the face nodes'
 // exterior values, then the reference (first node).
-template <int P, int STRIDE>
+template <int P, int Q, int STRIDE>
 __device__ __forceinline__ double* esdg_node_row(double* s_n, int le, int row) {
-  return s_n + (le * EsdgNodes<P, STRIDE>::ROWS + row) * STRIDE;
+  return s_n + (le * EsdgNodes<P, Q, STRIDE>::ROWS + row) * STRIDE;
 }
 
 // Fill them (fields of ev; extra(row, g) adds columns of its own for node g).
-template <int P, int NFLD, int STRIDE, typename Extra>
+template <int P, int Q, int NFLD, int STRIDE, typename Extra>
 __device__ __forceinline__ void esdg_load_nodes(const KArgs& a, const EsdgArgs& ea,
                                                 double* s_n, int64_t e0, int ne,
                                                 Extra extra) {
   using E = Elem<3, P>;
-  constexpr int NP = E::NP, NFN = E::NFN, ROWS = EsdgNodes<P, STRIDE>::ROWS;
+  constexpr int NP = E::NP, NFN = E::NFN, ROWS = EsdgNodes<P, Q, STRIDE>::ROWS;
   const int64_t N = a.nnodes;
   for (int t = threadIdx.x; t < ne * ROWS; t += kBlock) {
     const int le = t / ROWS;
@@ -428,7 +429,7 @@ __device__ __forceinline__ void esdg_load_nodes(const KArgs& a, const EsdgArgs& 
     if (r < NP) g = g0 + r;
     else if (r < NP + NFN) g = a.vmap_p[(e0 + le) * NFN + r - NP];
     if (g < 0) continue;   // boundary face node: not read
-    double* row = esdg_node_row<P, STRIDE>(s_n, le, r);
+    double* row = esdg_node_row<P, Q, STRIDE>(s_n, le, r);
     const bool first = r == NP + NFN;
 #pragma unroll
     for (int f = 0; f < NFLD; ++f) {
@@ -461,13 +462,13 @@ __device__ __forceinline__ void esdg_interp(const double* w, int ws, const doubl
 
 // {{{ ideal gas
 
-template <int P, int NSP>
+template <int P, int Q, int NSP>
 struct EsdgPairCfg {
-  using C = EsdgPairs<P, false>;
+  using C = EsdgPairs<Q, false>;
   static constexpr int NFLD = 5 + NSP;
   static constexpr int STRIDE = (NFLD + 1) / 2 * 2;
-  static constexpr int NODES = EsdgNodes<P, STRIDE>::SIZE;
-  static constexpr int PART = EsdgApply<P, false, NFLD>::PART;
+  static constexpr int NODES = EsdgNodes<P, Q, STRIDE>::SIZE;
+  static constexpr int PART = EsdgApply<P, Q, false, NFLD>::PART;
   static constexpr int POINTS = C::template POINTS<EcPair<3, NSP>> +
                                 C::EPB * (2 * C::NH + NFLD * C::NFT);
   static constexpr int ACC = C::EPB * NFLD * C::NACC;
@@ -547,12 +548,12 @@ __device__ __forceinline__ void ec_face_flux(const EcPrim<3, NSP>& m, const EcPr
 // ... at a boundary face point (quadrature point mm of face fc of element e):
 // the interpolated interior state, through the entropy variables and back as
 // the reference's projection does, and the condition's exterior state.
-template <int P, int NSP>
+template <int P, int Q, int NSP>
 __device__ __forceinline__ void ec_boundary_flux(const KArgs& a, const EsdgArgs& ea, int64_t e,
                                                  int fc, int mm, int32_t v0, const double* n,
                                                  double gamma, double sc, double* out) {
   using E = Elem<3, P>;
-  using C = EsdgPairs<P, false>;
+  using C = EsdgPairs<Q, false>;
   constexpr int NFLD = 5 + NSP;
   double ui[NFLD], vi[NFLD], qm[NFLD], qp[NFLD];
 #pragma unroll
@@ -581,13 +582,13 @@ __device__ __forceinline__ void ec_boundary_flux(const KArgs& a, const EsdgArgs&
   for (int f = 0; f < NFLD; ++f) out[f] = sc * (fs[f] - al * (qp[f] - qm[f]));
 }
 
-template <int P, int NSP>
+template <int P, int Q, int NSP>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(2))) void esdg_pair_kernel(KArgs a,
                                                                             EsdgArgs ea) {
   using E = Elem<3, P>;
-  using C = EsdgPairs<P, false>;
-  using Cfg = EsdgPairCfg<P, NSP>;
+  using C = EsdgPairs<Q, false>;
+  using Cfg = EsdgPairCfg<P, Q, NSP>;
   constexpr int NFLD = Cfg::NFLD, ST = Cfg::STRIDE, NH = C::NH, NFT = C::NFT;
   using Pt = EcPair<3, NSP>;
   extern __shared__ __align__(16) double lds16[];
@@ -599,11 +600,11 @@ __attribute__((amdgpu_waves_per_eu(2))) void esdg_pair_kernel(KArgs a,
   const int ne = a.K - e0 < C::EPB ? int(a.K - e0) : C::EPB;
   const double gamma = a.gas.gamma;
   // 1: projected entropy variables of the own and the neighbours' nodes
-  esdg_load_nodes<P, NFLD, ST>(a, ea, s_n, e0, ne, [](double*, int64_t) {});
+  esdg_load_nodes<P, Q, NFLD, ST>(a, ea, s_n, e0, ne, [](double*, int64_t) {});
   __syncthreads();
   if (int(threadIdx.x) < ne) {
     // the reference's v_0 becomes its density
-    double* r = esdg_node_row<P, ST>(s_n, threadIdx.x, E::NP + E::NFN);
+    double* r = esdg_node_row<P, Q, ST>(s_n, threadIdx.x, E::NP + E::NFN);
     const double w0 = -r[1];
     const double v2 = r[2] * r[2] + r[3] * r[3] + r[4] * r[4];
     r[0] = exp(r[0] + 0.5 * v2 / w0 - (gamma + log(w0)) / (gamma - 1.0));
@@ -617,10 +618,10 @@ __attribute__((amdgpu_waves_per_eu(2))) void esdg_pair_kernel(KArgs a,
     const int le = u / (face ? NFT : C::NQ);
     const int m = u - le * (face ? NFT : C::NQ);
     const int h = face ? C::NQ + m : m;
-    const double* ref = esdg_node_row<P, ST>(s_n, le, E::NP + E::NFN);
+    const double* ref = esdg_node_row<P, Q, ST>(s_n, le, E::NP + E::NFN);
     double d[NFLD];
     EcPrim<3, NSP> s;
-    esdg_interp<ST, NFLD, E::NP>(ea.vh + h, NH, esdg_node_row<P, ST>(s_n, le, 0), E::NP, d);
+    esdg_interp<ST, NFLD, E::NP>(ea.vh + h, NH, esdg_node_row<P, Q, ST>(s_n, le, 0), E::NP, d);
     ec_state<NSP>(ref, d, gamma, s);
     C::points(s_pt, le)[h] = s;
     s_log[2 * (le * NH + h)] = s.lrho;
@@ -637,21 +638,21 @@ __attribute__((amdgpu_waves_per_eu(2))) void esdg_pair_kernel(KArgs a,
     if (v0 >= 0) {
       EcPrim<3, NSP> p;
       esdg_interp<ST, NFLD, E::NFP>(ea.finterp + fc * E::NFP * C::NFQ + mm, C::NFQ,
-                                    esdg_node_row<P, ST>(s_n, le, E::NP + fc * E::NFP),
+                                    esdg_node_row<P, Q, ST>(s_n, le, E::NP + fc * E::NFP),
                                     E::NFP, d);
       ec_state<NSP>(ref, d, gamma, p);
       ec_face_flux<NSP>(s, p, n, gamma, ea.dissipation, sc, fs);
     } else {
-      ec_boundary_flux<P, NSP>(a, ea, e, fc, mm, v0, n, gamma, sc, fs);
+      ec_boundary_flux<P, Q, NSP>(a, ea, e, fc, mm, v0, n, gamma, sc, fs);
     }
 #pragma unroll
     for (int f = 0; f < NFLD; ++f) s_fs[(f * C::EPB + le) * NFT + m] = fs[f];
   }
   __syncthreads();
   // 3: rows of (Q_h - Q_h^T) o F_S, plus the face flux on face rows
-  esdg_pair_rows<P, false>(a, ea, EcPaired<3, NSP>(gamma), s_pt, s_log, 0, s_fs, lds16, e0, ne);
+  esdg_pair_rows<Q, false>(a, ea, EcPaired<3, NSP>(gamma), s_pt, s_log, 0, s_fs, lds16, e0, ne);
   // 4: dQ/dt = -M^-1 V_h^T acc
-  esdg_pair_apply<P, false, NFLD>(a, ea, lds16, s_n, e0, ne);
+  esdg_pair_apply<P, Q, false, NFLD>(a, ea, lds16, s_n, e0, ne);
 }
 
 // }}}
@@ -663,8 +664,8 @@ struct EsdgMixCfg {
   using C = EsdgPairs<P, true>;
   static constexpr int NFLD = 5 + MIX_NSP;
   static constexpr int STRIDE = NFLD + 2;   // + T, gamma(cv, T)
-  static constexpr int NODES = EsdgNodes<P, STRIDE>::SIZE;
-  static constexpr int PART = EsdgApply<P, true, NFLD>::PART;
+  static constexpr int NODES = EsdgNodes<P, P, STRIDE>::SIZE;
+  static constexpr int PART = EsdgApply<P, P, true, NFLD>::PART;
   static constexpr int POINTS =
       C::template POINTS<RnPoint<3>> + C::EPB * NFLD * C::NFT;
   static constexpr int ACC = C::EPB * NFLD * C::NACC;
@@ -774,7 +775,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void esdg_mix_pair_kernel(KArgs a, EsdgA
   const int ne = a.K - e0 < C::EPB ? int(a.K - e0) : C::EPB;
   // 1: projected entropy variables and T of the own and the neighbours'
   // nodes, gamma(cv, T) of the own
-  esdg_load_nodes<P, NFLD, ST>(a, ea, s_n, e0, ne, [&](double* row, int64_t g) {
+  esdg_load_nodes<P, P, NFLD, ST>(a, ea, s_n, e0, ne, [&](double* row, int64_t g) {
     row[IT] = a.temp[g];
   });
   if (int(threadIdx.x) < C::EPB) s_rng[threadIdx.x] = 3;
@@ -785,7 +786,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void esdg_mix_pair_kernel(KArgs a, EsdgA
 #pragma unroll
     for (int k = 0; k < MIX_NSP; ++k) y[k] = a.q[(5 + k) * a.nnodes + g] * irho;
     mix_temperature_poly(0.0, tn, y, 0, cvp, r);
-    esdg_node_row<P, ST>(s_n, t / E::NP, t % E::NP)[IG] = 1.0 + r / horner5(cvp, tn);
+    esdg_node_row<P, P, ST>(s_n, t / E::NP, t % E::NP)[IG] = 1.0 + r / horner5(cvp, tn);
   }
   __syncthreads();
   double tmid_lo, tmid_hi;
@@ -829,12 +830,12 @@ __attribute__((amdgpu_waves_per_eu(2))) void esdg_mix_pair_kernel(KArgs a, EsdgA
         sc = a.fscale[e * 4 + fc] * ea.wf[mm];
       }
       if (v0 >= 0) {
-        const double* ref = esdg_node_row<P, ST>(s_n, le, E::NP + E::NFN);
+        const double* ref = esdg_node_row<P, P, ST>(s_n, le, E::NP + E::NFN);
         double d[NFLD + 2];
         const double* w = nbr ? ea.finterp + fc * E::NFP * C::NFQ + mm : ea.vh + h;
         esdg_interp<ST, NFLD + 2, E::NP>(
             w, nbr ? C::NFQ : NH,
-            esdg_node_row<P, ST>(s_n, le, nbr ? E::NP + fc * E::NFP : 0),
+            esdg_node_row<P, P, ST>(s_n, le, nbr ? E::NP + fc * E::NFP : 0),
             nbr ? E::NFP : E::NP, d);
         if (!nbr) gh = d[IG];   // the neighbour's state takes this side's gamma
         RnState s;
@@ -896,7 +897,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void esdg_mix_pair_kernel(KArgs a, EsdgA
     esdg_pair_rows<P, true>(a, ea, RnPaired<3, false>(own_poly), s_pt, nullptr, LOG0, s_fs, lds16,
                             e0, ne);
   // 4: dQ/dt = -M^-1 V_h^T acc
-  esdg_pair_apply<P, true, NFLD>(a, ea, lds16, s_n, e0, ne);
+  esdg_pair_apply<P, P, true, NFLD>(a, ea, lds16, s_n, e0, ne);
 }
 
 // }}}

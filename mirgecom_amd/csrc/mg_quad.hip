@@ -119,17 +119,15 @@ mg_status esdg_check(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* quad
 constexpr size_t kEsdgBudget = 128 * 1024;
 
 // The paired flux-differencing kernels (mg_esdg_pairs.h) take 3-D elements
-// with the default quadrature (their lane layout is its point counts) and the
+// whose rule has (Q+1)^3 and 3 (Q+1)^2 points (their lane layout) and the
 // operators' cyclic diagonals; any other rule goes row by row, which evaluates
-// nearly every two-point flux twice.
-template <int D, int P>
+// nearly every two-point flux twice.  Q = p is the default rule; without a
+// mixture p = 1 and 2 also take the 64-point rule of degree 6 and 7 (p = 2,
+// 1,296 tets: 96 us, row by row 232).
+template <int Q>
 bool esdg_paired(const mgdg::EsdgArgs& ea) {
-  if constexpr (D == 3) {
-    using C = mgdg::EsdgPairs<P, false>;
-    return ea.skew_diag && ea.ext_diag && ea.nq == C::NQ && ea.nfq == C::NFQ;
-  } else {
-    return false;
-  }
+  using C = mgdg::EsdgPairs<Q, false>;
+  return ea.skew_diag && ea.ext_diag && ea.nq == C::NQ && ea.nfq == C::NFQ;
 }
 
 template <typename Kern>
@@ -161,6 +159,13 @@ mg_status esdg_launch_rows(Kern kern, const char* name, size_t per, const mgdg::
   return esdg_launch_one(kern, name, per * epb, kEsdgBudget, epb, a, ea, st);
 }
 
+template <int P, int Q, int NS>
+mg_status esdg_launch_paired(const mgdg::KArgs& a, mgdg::EsdgArgs& ea, hipStream_t st) {
+  constexpr size_t lds = mgdg::EsdgPairCfg<P, Q, NS>::LDS;
+  return esdg_launch_one(mgdg::esdg_pair_kernel<P, Q, NS>, "esdg_pair_kernel", lds, lds,
+                         mgdg::EsdgPairs<Q, false>::EPB, a, ea, st);
+}
+
 template <int D, int P, int NS>
 mg_status esdg_launch(const mgdg::KArgs& a, mgdg::EsdgArgs& ea, hipStream_t st) {
   using E = mgdg::Elem<D, P>;
@@ -168,11 +173,8 @@ mg_status esdg_launch(const mgdg::KArgs& a, mgdg::EsdgArgs& ea, hipStream_t st) 
                                     "esdg_project_kernel", 2 + D + NS, a, ea, st);
   if (s) return s;
   if constexpr (D == 3) {
-    if (esdg_paired<D, P>(ea)) {
-      constexpr size_t lds = mgdg::EsdgPairCfg<P, NS>::LDS;
-      return esdg_launch_one(mgdg::esdg_pair_kernel<P, NS>, "esdg_pair_kernel", lds, lds,
-                             mgdg::EsdgPairs<P, false>::EPB, a, ea, st);
-    }
+    if (esdg_paired<P>(ea)) return esdg_launch_paired<P, P, NS>(a, ea, st);
+    if (esdg_paired<3>(ea)) return esdg_launch_paired<P, 3, NS>(a, ea, st);
   }
   const size_t nq = ea.nq, nft = size_t(D + 1) * ea.nfq, nh = ea.nh;
   const size_t nacc = (nh + nq - 1) / nq * nq + nft;
@@ -189,7 +191,7 @@ mg_status esdg_mix_launch(const mgdg::KArgs& a, mgdg::EsdgArgs& ea, hipStream_t 
                                     "esdg_project_mix_kernel", NF, a, ea, st);
   if (s) return s;
   if constexpr (D == 3) {
-    if (esdg_paired<D, P>(ea)) {
+    if (esdg_paired<P>(ea)) {
       constexpr size_t lds = mgdg::EsdgMixCfg<P>::LDS;
       return esdg_launch_one(mgdg::esdg_mix_pair_kernel<P>, "esdg_mix_pair_kernel", lds, lds,
                              mgdg::EsdgPairs<P, true>::EPB, a, ea, st);
