@@ -37,9 +37,10 @@ namespace mgdg {
 // same volume point, which is then read from LDS once and moved once per step
 // for RT fluxes) and each block's steps are cut into NC = 4/NB pieces; the
 // volume rows' steps are cut into four.  Every slot so has the same work.
-// RT as large as the registers of two waves per SIMD hold: for the 12-field
-// mixture at p = 2 two rows per lane spilled in the loop and took 1.31 ms
-// where one takes 1.25; three waves per SIMD for the ideal gas spilled and
+// RT as large as the registers hold: of two waves per SIMD where two
+// workgroups share a CU's LDS (the ideal gas, and 12 fields at p = 2: for the
+// mixture two rows per lane spilled in the loop there and took 1.31 ms where
+// one takes 1.25; three waves per SIMD for the ideal gas spilled and
 // took 7.5 ms.  The sums stay in registers until all of the
 // workgroup's pairs are done and then go over the points' LDS: four pieces
 // of the volume rows, NC of the face rows, added before the last phase.
@@ -383,6 +384,13 @@ __device__ __forceinline__ void esdg_pair_apply(const KArgs& a, const EsdgArgs& 
   }
 }
 
+// Waves per SIMD to plan the registers for: two where two workgroups fit a CU's
+// LDS, all registers for one otherwise (12 fields at Q = 1 and 3: with the
+// registers of two they spilled up to 330; mixture p = 1, 24,576 tets 723 -> 413
+// us, p = 3, 6,000 tets 2541 -> 1143; passive species p = 1 374 -> 250, p = 3
+// 1502 -> 855).
+constexpr int esdg_waves(size_t lds) { return lds <= 80 * 1024 ? 2 : 1; }
+
 // }}}
 
 // {{{ states at the hybridized points
@@ -584,8 +592,8 @@ __device__ __forceinline__ void ec_boundary_flux(const KArgs& a, const EsdgArgs&
 
 template <int P, int Q, int NSP>
 __global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(2))) void esdg_pair_kernel(KArgs a,
-                                                                            EsdgArgs ea) {
+__attribute__((amdgpu_waves_per_eu(esdg_waves(EsdgPairCfg<P, Q, NSP>::LDS)))) void
+esdg_pair_kernel(KArgs a, EsdgArgs ea) {
   using E = Elem<3, P>;
   using C = EsdgPairs<Q, false>;
   using Cfg = EsdgPairCfg<P, Q, NSP>;
@@ -757,7 +765,8 @@ __device__ __forceinline__ void rn_boundary_flux(const KArgs& a, const EsdgArgs&
 
 template <int P>
 __global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(2))) void esdg_mix_pair_kernel(KArgs a, EsdgArgs ea) {
+__attribute__((amdgpu_waves_per_eu(esdg_waves(EsdgMixCfg<P>::LDS)))) void
+esdg_mix_pair_kernel(KArgs a, EsdgArgs ea) {
   using E = Elem<3, P>;
   using C = EsdgPairs<P, true>;
   using Cfg = EsdgMixCfg<P>;
