@@ -35,23 +35,40 @@ mg_status quad_ns_check(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* q
 // LDS row strides = 4 mod 32 doubles (bank spread of the matrix-core reads)
 int bank_stride(int n) { return n + ((4 - n % 32) + 32) % 32; }
 
-// Elements per workgroup: as many (at most 16) as leave room for two
-// workgroups on a CU (80 KiB each), at least one; one element may take up to
-// 128 KiB.
+// Elements per workgroup: at most 16, as many as leave room for two workgroups
+// on a CU (80 KiB each); at least one, which may take up to 128 KiB.
 constexpr size_t kQuadBudget = 128 * 1024;
 
-template <typename Kern, typename Lds>
-mg_status quad_launch(Kern kern, Lds lds, const char* name, const mgdg::KArgs& a,
-                      mgdg::QuadArgs& qa, hipStream_t st) {
-  auto bytes = [&](int epb) { return sizeof(double) * lds(qa.gs, qa.fs, epb); };
-  if (bytes(1) > kQuadBudget) return fail(MG_ERR_UNSUPPORTED, "quadrature too large for LDS");
+template <typename Lds>
+int quad_epb(Lds lds, const mgdg::QuadArgs& qa) {
   int epb = 1;
-  while (epb < 16 && bytes(epb + 1) <= 80 * 1024) ++epb;
+  while (epb < 16 && sizeof(double) * lds(qa.gs, qa.fs, epb + 1) <= 80 * 1024) ++epb;
+  return epb;
+}
+
+// ... of those, where the contraction takes rounds(epb) rounds of the four
+// waves, the number with the fewest rounds per element, the largest on a tie.
+// Gradients of the ideal gas, MI355X, tets: p = 1, 131,712 392 -> 335 us (14 ->
+// 10 elements: 84 columns are six tiles of 16 and two rounds, 60 four and one);
+// p = 4, 10,368 400 -> 335 us (3 -> 2); triangles, p = 1, 4,608 14.9 -> 12.4 us.
+template <typename Rounds>
+int quad_epb_rounds(int most, Rounds rounds) {
+  int epb = 1;
+  for (int n = 2; n <= most; ++n)
+    if (rounds(n) * epb <= rounds(epb) * n) epb = n;
+  return epb;
+}
+
+template <typename Kern, typename Lds>
+mg_status quad_launch(Kern kern, Lds lds, int epb, const char* name, const mgdg::KArgs& a,
+                      mgdg::QuadArgs& qa, hipStream_t st) {
+  const size_t bytes = sizeof(double) * lds(qa.gs, qa.fs, epb);
+  if (bytes > kQuadBudget) return fail(MG_ERR_UNSUPPORTED, "quadrature too large for LDS");
   qa.epb = epb;
   mg_status s = set_lds(kern, kQuadBudget);
   if (s) return s;
-  hipLaunchKernelGGL(kern, dim3(unsigned((a.K + epb - 1) / epb)), dim3(mgdg::kBlock),
-                     bytes(epb), st, a, qa);
+  hipLaunchKernelGGL(kern, dim3(unsigned((a.K + epb - 1) / epb)), dim3(mgdg::kBlock), bytes, st,
+                     a, qa);
   return check_launch(name);
 }
 

@@ -24,9 +24,13 @@ mg_status mg_ns_gradient_quad(const mg_mesh* mesh, const mg_gas* gas, const mg_q
   hipStream_t st = static_cast<hipStream_t>(stream);
 #define MG_GCASE(D, P, NS, MX)                                                      \
   if (mesh->dim == D && mesh->order == P && gas->nspecies == NS && var == MX) {     \
-    return quad_launch(mgdg::ns_grad_quad_kernel<D, P, NS, MX>,                     \
-                       mgdg::quad_grad_lds<D, P, NS, MX>, "ns_grad_quad_kernel", a, \
-                       qa, st);                                                     \
+    constexpr auto lds = mgdg::quad_grad_lds<D, P, NS, MX>;                         \
+    auto rounds = [](int epb) {                                                     \
+      return (mgdg::quad_tiles(mgdg::Elem<D, P>::NP, (3 + D + NS) * epb) + 3) / 4;  \
+    };                                                                              \
+    return quad_launch(mgdg::ns_grad_quad_kernel<D, P, NS, MX>, lds,                \
+                       quad_epb_rounds(quad_epb(lds, qa), rounds),                  \
+                       "ns_grad_quad_kernel", a, qa, st);                           \
   }
   MG_NSQ_CASES(MG_GCASE)
 #undef MG_GCASE

@@ -29,9 +29,9 @@ mg_status mg_ns_rhs_quad(const mg_mesh* mesh, const mg_gas* gas, const mg_quad* 
   hipStream_t st = static_cast<hipStream_t>(stream);
 #define MG_DCASE(D, P, NS, MX)                                                      \
   if (mesh->dim == D && mesh->order == P && gas->nspecies == NS && var == MX) {     \
-    return quad_launch(mgdg::ns_div_quad_kernel<D, P, NS, MX>,                      \
-                       mgdg::quad_div_lds<D, P, NS, MX>, "ns_div_quad_kernel", a,   \
-                       qa, st);                                                     \
+    constexpr auto lds = mgdg::quad_div_lds<D, P, NS, MX>;                          \
+    return quad_launch(mgdg::ns_div_quad_kernel<D, P, NS, MX>, lds,                 \
+                       quad_epb(lds, qa), "ns_div_quad_kernel", a, qa, st);         \
   }
   MG_NSQ_CASES(MG_DCASE)
 #undef MG_DCASE

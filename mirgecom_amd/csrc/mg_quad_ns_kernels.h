@@ -37,16 +37,17 @@ namespace mgdg {
 // two columns each: at the matrix cores' rate, one wave's keep LDS busy for as
 // long as its products take, and the four SIMDs share it.  Ideal gas, p = 3,
 // 82,944 elements, 64 volume and 48 face points: divergence 2194 -> 1317 us;
-// mixture, p = 2, 24,576 elements: 1057 -> 1000 us.  (The gradient, 5 columns,
-// stays at 880 us: its contraction takes as long as its points.)  2-D faces
-// have p + 1 points, which would leave most of a tile empty: there the lanes
-// keep reading the columns, several nodes per step, the next step's weights and
-// face nodes already on their way.  ST is 2 mod 4 doubles, which spreads the
-// node-by-node writes over the LDS banks.
+// mixture, p = 2, 24,576 elements: 1057 -> 1000 us.  2-D faces have p + 1
+// points, which would leave most of a tile empty, and the ideal gas's gradient
+// has 5 columns (p = 1, 6,000 to 384,000 elements: the products take 4 % longer;
+// p = 3, 4 alike): there the lanes keep reading the columns, several nodes per
+// step, the next step's weights and face nodes already on their way.  ST is 2
+// mod 4 doubles, which spreads the node-by-node writes over the LDS banks.
 template <int DIM, int P, int NSP, int MIX, bool GRAD>
 struct QuadNs {
   using E = Elem<DIM, P>;
-  static constexpr bool MM = DIM == 3;   // interpolation on the matrix cores
+  // interpolation on the matrix cores
+  static constexpr bool MM = DIM == 3 && (GRAD || NSP > 0);
   static constexpr int NFLD = 2 + DIM + NSP, NS = NFLD + 1, NSD = NS * DIM;
   static constexpr int NQC = NFLD + (MIX != 0 ? 1 : 0);
   static constexpr int NG = NSD - DIM;   // the viscous flux takes no energy gradient
@@ -403,10 +404,11 @@ __device__ __forceinline__ int quad_task_count(int groups, int n) {
 __device__ __forceinline__ int quad_first_task() {
   return (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + (blockIdx.x >> 3)) & (kWaves - 1);
 }
-// The lane's point of a task; 2-D: 64 consecutive points, at most one tile.
-template <int DIM, int P>
+// The lane's point of a task; without tiles 64 consecutive points, at most one
+// past the last.
+template <int DIM, int P, bool MM>
 __device__ __forceinline__ QuadTiles<DIM, P> quad_point(bool face, int task, int ne, int n) {
-  if constexpr (DIM == 3) {
+  if constexpr (MM) {
     return QuadTiles<DIM, P>(face, task, ne, n);
   } else {
     QuadTiles<DIM, P> tl;
@@ -452,7 +454,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void ns_grad_quad_kernel(KArgs a, QuadAr
   const int ntask = nvt + quad_task_count<C::MM>(ne * NF, nfq);
   for (int task = quad_first_task(); task < ntask; task += kWaves) {
     const bool face = task >= nvt;
-    const auto tl = quad_point<DIM, P>(face, face ? task - nvt : task, ne, face ? nfq : nq);
+    const auto tl = quad_point<DIM, P, C::MM>(face, face ? task - nvt : task, ne, face ? nfq : nq);
     if (!C::MM && !tl.valid) continue;
     const int le = tl.le, m = tl.m;
     const double* rows = s_n + le * C::ROWS * ST;
@@ -606,7 +608,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void ns_div_quad_kernel(KArgs a, QuadArg
   const int ntask = nvt + quad_task_count<C::MM>(ne * NF, nfq);
   for (int task = quad_first_task(); task < ntask; task += kWaves) {
     const bool face = task >= nvt;
-    const auto tl = quad_point<DIM, P>(face, face ? task - nvt : task, ne, face ? nfq : nq);
+    const auto tl = quad_point<DIM, P, C::MM>(face, face ? task - nvt : task, ne, face ? nfq : nq);
     if (!C::MM && !tl.valid) continue;
     const int le = tl.le, m = tl.m;
     const double* rows = s_n + le * C::ROWS * ST;
