@@ -83,13 +83,14 @@ def _nasa7(t, coef_lo, coef_hi):
     return cp, h, s
 
 
-def source_buffer(q, dim):
-    """A buffer like ``q`` for species sources, zero outside the mechanism's
+def source_buffer(q, dim, n):
+    """A buffer like ``q`` (``n`` nodes) for species sources, zero outside the mechanism's
     species rows, every one of which the source kernels write.  From 2**17 nodes
     on only the zero rows are filled, 15 us less at 1.97 M nodes; below, where
     the host's calls count, one fill of everything saves two of them, 1 us of
-    78.  A state with further rows is filled whole too."""
-    if q.numel() < q.shape[0] << 17 or q.shape[0] != 2 + dim + mech.NSPECIES:
+    78 (and the comparison must stay cheap: looking up the state's shape for it
+    cost 0.6 us of 60).  A state with further rows is filled whole too."""
+    if n < 1 << 17 or q.shape[0] != 2 + dim + mech.NSPECIES:
         return torch.zeros_like(q)
     out = torch.empty_like(q)
     out[:2 + dim].zero_()
@@ -223,8 +224,8 @@ class PyrometheusMixture:
         from mirgecom_amd.fluid import ConservedVars
         q = cv.q.contiguous()
         t = temperature.contiguous()
-        out = source_buffer(q, cv.dim)
         n = cv.mass.numel()
+        out = source_buffer(q, cv.dim, n)
         _lib.ensure_mechanism()
         gas = _lib.MgGas(eos_kind=1, nspecies=7)
         _lib.call("mg_species_source", gas, cv.dim, n, _lib.ptr(q), _lib.ptr(t),

@@ -20,7 +20,7 @@ def test_zero_rows(monkeypatch, nodes, dim, extra):
     from mirgecom_amd.eos import source_buffer
     _poison(monkeypatch)
     q = torch.ones((9 + dim + extra, nodes, 1), dtype=torch.float64)
-    out = source_buffer(q, dim)
+    out = source_buffer(q, dim, nodes)
     assert out.shape == q.shape and out.dtype == q.dtype and out.is_contiguous()
     assert nodes == 0 or out.data_ptr() != q.data_ptr()
     assert (out[:2 + dim] == 0).all()
