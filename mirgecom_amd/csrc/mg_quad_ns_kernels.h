@@ -578,9 +578,19 @@ __attribute__((amdgpu_waves_per_eu(2))) void ns_grad_quad_kernel(KArgs a, QuadAr
   }
 }
 
+// Waves per SIMD that the divergence's registers are planned for.  Two spill 100
+// to 280 VGPRs with species, one none; which is faster as measured, MI355X,
+// mixture, two -> one: 2-D p = 1..4, 4,608 triangles 28, 48, 53, 77 -> 33, 53,
+// 58, 96 us; 3-D p = 1, 131,712 tets 2.71 -> 2.35 ms, p = 2 5.54 -> 5.74 ms,
+// p = 3, 10,368 0.79 -> 0.73 ms, p = 4 (one workgroup fills a CU's LDS) 2.56 ->
+// 1.62 ms.
+constexpr int quad_div_waves(int dim, int p, int nsp) {
+  return dim == 3 && p != 2 && nsp > 0 ? 1 : 2;
+}
+
 template <int DIM, int P, int NSP, int MIX>
 __global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(2))) void ns_div_quad_kernel(KArgs a, QuadArgs qa) {
+__attribute__((amdgpu_waves_per_eu(quad_div_waves(DIM, P, NSP)))) void ns_div_quad_kernel(KArgs a, QuadArgs qa) {
   using E = Elem<DIM, P>;
   using C = QuadNs<DIM, P, NSP, MIX, true>;
   constexpr int NP = E::NP, NFP = E::NFP, NF = E::NF, ST = C::ST;
