@@ -46,11 +46,13 @@ int quad_epb(Lds lds, const mgdg::QuadArgs& qa) {
   return epb;
 }
 
-// ... of those, where the contraction takes rounds(epb) rounds of the four
-// waves, the number with the fewest rounds per element, the largest on a tie.
-// Gradients of the ideal gas, MI355X, tets: p = 1, 131,712 392 -> 335 us (14 ->
-// 10 elements: 84 columns are six tiles of 16 and two rounds, 60 four and one);
-// p = 4, 10,368 400 -> 335 us (3 -> 2); triangles, p = 1, 4,608 14.9 -> 12.4 us.
+// ... of those, the number with the fewest rounds(epb) of the four waves per
+// element (tasks of points, and twice the contraction's tiles, one of whose rounds
+// takes about as long as two of points), the largest on a tie.  Gradients, MI355X,
+// the largest number -> this: ideal gas, tets, p = 1, 131,712 392 -> 335 us (14 ->
+// 10 elements: 84 columns are six tiles of 16 and two rounds, 60 four and one),
+// p = 4, 10,368 400 -> 334 us (3 -> 2), p = 2, 10,368 63 -> 55 us (8 -> 7), p = 3
+// unchanged (5); mixture, 4,608 triangles, p = 4 44 -> 34 us.
 template <typename Rounds>
 int quad_epb_rounds(int most, Rounds rounds) {
   int epb = 1;

@@ -25,8 +25,12 @@ mg_status mg_ns_gradient_quad(const mg_mesh* mesh, const mg_gas* gas, const mg_q
 #define MG_GCASE(D, P, NS, MX)                                                      \
   if (mesh->dim == D && mesh->order == P && gas->nspecies == NS && var == MX) {     \
     constexpr auto lds = mgdg::quad_grad_lds<D, P, NS, MX>;                         \
-    auto rounds = [](int epb) {                                                     \
-      return (mgdg::quad_tiles(mgdg::Elem<D, P>::NP, (3 + D + NS) * epb) + 3) / 4;  \
+    auto rounds = [&](int epb) {                                                    \
+      using C = mgdg::QuadNs<D, P, NS, MX, false>;                                  \
+      const int tasks = mgdg::quad_task_count<C::MM>(epb, qa.nq) +                  \
+                        mgdg::quad_task_count<C::MM>((D + 1) * epb, qa.nfq);        \
+      const int tiles = mgdg::quad_tiles(mgdg::Elem<D, P>::NP, (3 + D + NS) * epb);  \
+      return (tasks + 3) / 4 + 2 * ((tiles + 3) / 4);                               \
     };                                                                              \
     return quad_launch(mgdg::ns_grad_quad_kernel<D, P, NS, MX>, lds,                \
                        quad_epb_rounds(quad_epb(lds, qa), rounds),                  \

@@ -398,7 +398,7 @@ __device__ __forceinline__ double quad_point_temperature(const double* q, double
 // block, so that two workgroups on a CU do not both give their surplus task to
 // the same SIMD.
 template <bool MM>
-__device__ __forceinline__ int quad_task_count(int groups, int n) {
+__host__ __device__ __forceinline__ int quad_task_count(int groups, int n) {
   return MM ? (groups * ((n + 15) / 16) + 3) / 4 : (groups * n + 63) / 64;
 }
 __device__ __forceinline__ int quad_first_task() {
