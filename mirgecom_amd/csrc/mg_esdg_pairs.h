@@ -4,14 +4,14 @@
 // once, for both of its rows; other rules and 2-D take the row-by-row kernels
 // (mgdg_kernels.h).
 //
-// Measured on an MI355X (kernel with the projection, before -> after this
-// layout): ideal gas p = 3, 82,944 tets 6.1 -> 4.4 ms; uiuc_7sp mixture
-// p = 2, 24,576 tets 4.35 -> 1.25 ms (the row-by-row kernel evaluates 6,561
-// fluxes per element, this one 3,267); p = 1 mixture, 15,288 tets
-// 0.64 -> 0.24 ms.  The ideal gas is bound by FP64 VALU issue (67 % of the
-// cycles with two waves per SIMD), half of it in the pair loop, the rest in
-// the states and the contraction; the mixture by LDS (64 % busy) and VALU
-// (52 %).
+// Measured on an MI355X (kernel with the projection, row by row -- ideal gas
+// p = 3: an earlier paired kernel -- -> this layout): ideal gas p = 3, 82,944 tets
+// 6.33 -> 4.39 ms; uiuc_7sp mixture p = 2, 24,576 tets 4.37 -> 1.14 ms (the
+// row-by-row kernel evaluates 6,561 fluxes per element, this one 3,267); p = 1,
+// 15,288 tets 0.92 -> 0.28 ms; p = 3, 6,000 tets 3.08 -> 1.15 ms.  The ideal gas is
+// bound by FP64 VALU issue (busy 70 % of the cycles with two waves per SIMD; LDS
+// 32 %), half of it in the pair loop, the rest in the states and the contraction;
+// the mixture at p = 2 by LDS (70 % busy) and VALU (51 %).
 #pragma once
 #include <cstddef>
 #include <type_traits>
@@ -39,8 +39,8 @@ namespace mgdg {
 // volume rows' steps are cut into four.  Every slot so has the same work.
 // RT as large as the registers hold: of two waves per SIMD where two
 // workgroups share a CU's LDS (the ideal gas, and 12 fields at p = 2: for the
-// mixture two rows per lane spilled in the loop there and took 1.31 ms where
-// one takes 1.25; three waves per SIMD for the ideal gas spilled and
+// mixture two rows per lane spilled in the loop there and took 5 % longer
+// than one; three waves per SIMD for the ideal gas spilled and
 // took 7.5 ms.  The sums stay in registers until all of the
 // workgroup's pairs are done and then go over the points' LDS: four pieces
 // of the volume rows, NC of the face rows, added before the last phase.

@@ -477,7 +477,7 @@ static __global__ __launch_bounds__(256) void adam_kernel(float* __restrict__ pr
 // exact rates (mix_species_source).
 //
 // Bound by the vector units (GELU is 60 % of their instructions) and the matrix
-// cores after each other: the first are busy 64 %, the second 27 % of the
+// cores after each other: the first are busy 60 %, the second 25 % of the
 // time.  1.97 M nodes, np = 10: 1282 us with an 8-operation GELU, the bias
 // added behind it and the sampled check at the end; 1116 us with GELU in 5,
 // the sums started from the bias and the check moved beside the features;
