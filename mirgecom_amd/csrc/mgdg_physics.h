@@ -654,6 +654,10 @@ struct EcPairLog : EcSpecies<NSP> {
   double uh[DIM];  // u / 2
 };
 
+static_assert(sizeof(EcPairLog<3, 0>) == 9 * 8 && sizeof(EcPairLog<3, 7>) == 15 * 8 &&
+                  sizeof(EcPairLog<2, 7>) == 14 * 8,
+              "LDS bank spread of the row-by-row kernels' points");
+
 // ... with the pressure and the wavespeed |u| + c the face flux needs.
 template <int DIM, int NSP>
 struct EcPrim : EcPairLog<DIM, NSP> {
